@@ -397,6 +397,7 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g2.A = h; g2.lda = d.I; g2.a_rows = d.T; g2.B0 = ptrs + 2 * d.E; g2.ldb = d.I; g2.kseg = d.I;
   g2.N = d.D; g2.K = d.I; g2.C = y_sorted; g2.ldc = d.D;
   const bool mfr = gemm_mfma_eligible(g, d.dtype, mf) && gemm_mfma_eligible(g2, d.dtype, mf);
+  const bool al = d.dtype == DSMOE_F32 ? mf : mfr;
   const int bm = gemm_tile_m(mfr);
   rc = launch_sched_from_offsets(offsets, d.E, bm, d.T, off32, sched, cnt, st);
   if (rc) return rc;
@@ -404,9 +405,9 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g.sched_count = g2.sched_count = cnt;
   g.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(d.T, d.E, bm);
   g.bm = g2.bm = bm;
-  rc = launch_grouped_gemm(g, EPI_SWIGLU, d.dtype, nullptr, mfr, st);
+  rc = launch_grouped_gemm(g, EPI_SWIGLU, d.dtype, nullptr, al, st);
   if (rc) return rc;
-  return launch_grouped_gemm(g2, EPI_STORE, d.dtype, sorted_w, mfr, st);
+  return launch_grouped_gemm(g2, EPI_STORE, d.dtype, sorted_w, al, st);
 }
 
 int dsmoe_combine_fwd(const void* o_slots, const float* weights, const int32_t* idx, const void* shared,
@@ -485,6 +486,7 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   // combine and the backward read slot s at row slot_pos[s]
   g2.N = d.D; g2.K = d.I; g2.C = L.o_sorted; g2.ldc = d.D;
   const bool mfr = gemm_mfma_eligible(g1, d.dtype, mf) && gemm_mfma_eligible(g2, d.dtype, mf);
+  const bool al = d.dtype == DSMOE_F32 ? mf : mfr;
   // Decode shapes (at most SK_MAX_T tokens, inference): every routed and
   // shared row tile fits the few-row kernel, which streams the weights once.
   bool sk = false;
@@ -542,8 +544,8 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   if (sk) g1.Gs = g1.Us = s1.Gs = s1.Us = nullptr;  // inference: no pre-activation saves
   tm.begin(ST_GEMM1);
   rc = sk ? launch_sk_pair(g1, s1, d.S > 0, EPI_SWIGLU, d.dtype, mf, st)
-          : d.S ? launch_grouped_gemm_pair(g1, s1, EPI_SWIGLU, d.dtype, nullptr, mfr, mf, st)
-                : launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, mfr, st);
+          : d.S ? launch_grouped_gemm_pair(g1, s1, EPI_SWIGLU, d.dtype, nullptr, al, mf, st)
+                : launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, al, st);
   tm.end();
   if (rc) return rc;
   // down projections: routed rows written in expert-sorted order (row r of
@@ -551,8 +553,8 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   // at row slot_pos[s]
   tm.begin(ST_GEMM2);
   rc = sk ? launch_sk_pair(g2, s2, d.S > 0, EPI_STORE, d.dtype, mf, st)
-          : d.S ? launch_grouped_gemm_pair(g2, s2, EPI_STORE, d.dtype, nullptr, mfr, mf, st)
-                : launch_grouped_gemm(g2, EPI_STORE, d.dtype, nullptr, mfr, st);
+          : d.S ? launch_grouped_gemm_pair(g2, s2, EPI_STORE, d.dtype, nullptr, al, mf, st)
+                : launch_grouped_gemm(g2, EPI_STORE, d.dtype, nullptr, al, st);
   tm.end();
   if (rc) return rc;
   // (d) combine
@@ -589,7 +591,7 @@ struct BwdLayout {
   void* dgdu_s;       // (T, 2 S I_s)
   void* dx_shared;    // (T, D)
   void* dy_w;         // bf16: (N, D) w * dY in sorted order (K-major operand of dW2)
-  int ks13, ks2;      // split-K of the shared-expert weight gradients (bf16 MFMA path)
+  int ks13, ks2;      // split-K of the shared-expert weight gradients
   float* part;        // fp32 split-K partials, max(ks13 * 2 I_s, ks2 * I_s) * S * D
   size_t total;
 };
@@ -637,9 +639,14 @@ static BwdLayout bwd_layout(const dsmoe_dims& d, void* base) {
   B.dy_w = (d.dtype == DSMOE_BF16 && d.D % 8 == 0) ? c.take<char>((size_t)N * d.D * es) : nullptr;
   B.ks13 = B.ks2 = 1;
   B.part = nullptr;
-  if (d.S && d.dtype == DSMOE_BF16) {
-    B.ks13 = xgemm_pick_ksplit(xgemm_tiles(2 * (int64_t)d.I_s, d.D, d.S), d.T);
-    B.ks2 = xgemm_pick_ksplit(xgemm_tiles(d.D, d.I_s, d.S), d.T);
+  if (d.S) {
+    if (d.dtype == DSMOE_BF16) {
+      B.ks13 = xgemm_pick_ksplit(xgemm_tiles(2 * (int64_t)d.I_s, d.D, d.S), d.T);
+      B.ks2 = xgemm_pick_ksplit(xgemm_tiles(d.D, d.I_s, d.S), d.T);
+    } else {
+      B.ks13 = xgemm_f32_ksplit(2 * (int64_t)d.I_s, d.D, d.S, d.T);
+      B.ks2 = xgemm_f32_ksplit(d.D, d.I_s, d.S, d.T);
+    }
     const int64_t n13 = B.ks13 > 1 ? (int64_t)B.ks13 * 2 * d.I_s : 0;
     const int64_t n2 = B.ks2 > 1 ? (int64_t)B.ks2 * d.I_s : 0;
     const int64_t nmax = std::max(n13, n2);
@@ -955,7 +962,7 @@ int dsmoe_grouped_swiglu_bwd(const void* x_sorted, const void* const* w1, const 
   // recompute g = X W1^T, u = X W3^T, h = silu(g) * u
   g1.B0 = B.w1; g1.B1 = B.w3; g1.C = B.h; g1.Gs = B.g; g1.Us = B.u;
   g1.sched = B.sched_f; g1.sched_count = B.cnt_f; g1.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm_f); g1.bm = bm_f;
-  rc = launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, mfr, st);
+  rc = launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, d.dtype == DSMOE_F32 ? mf : mfr, st);
   if (rc) return rc;
   const int32_t mbound = (int32_t)sched_bound(N, d.E, BWD_BM);
   // dh = dY W2, SwiGLU backward -> [dg | du]

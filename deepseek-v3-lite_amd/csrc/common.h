@@ -124,7 +124,7 @@ struct GemmDesc {
   void* Us;
 };
 
-constexpr int TILE_M = 128;   // M tile of the SIMT fallback GEMM
+constexpr int TILE_M = 128;   // M tile of the schedules of the SIMT and fp32 GEMMs
 constexpr int MAX_TOPK = 16;
 
 struct GateOut {
@@ -210,7 +210,8 @@ int launch_gather_rows(const void* x, int64_t src_rows, const int32_t* rows, int
                        hipStream_t st);
 int launch_sched_from_offsets(const int64_t* offsets64, int E, int bm, int64_t rows, int32_t* offsets32, MTile* sched,
                               int32_t* sched_count, hipStream_t st);
-// Whether launch_grouped_gemm will take the MFMA kernel for this descriptor,
+struct XGemm;
+// Whether launch_grouped_gemm will take the bf16 MFMA kernel for this descriptor,
 // and the M-tile height of that choice; the routed schedule (and desc.bm) must
 // be built with the same height.
 bool gemm_mfma_eligible(const GemmDesc& g, int dtype, bool allow_mfma);
@@ -220,6 +221,14 @@ int launch_gemm_qp(const GemmDesc& g, int epi, const float* row_scale, hipStream
 int launch_gemm_qp_pair(const GemmDesc& gr, const GemmDesc& gd, int epi, const float* row_scale, hipStream_t st);
 int launch_grouped_gemm(const GemmDesc& g, int epi, int dtype, const float* row_scale, bool allow_mfma,
                         hipStream_t st);
+// fp32 problems on the fp32 matrix cores (gemm_f32.hip), any shape and stride:
+// gr, and gd (dense, optional) in the same launch; row_scale applies to gr.
+// tables_aligned: every weight (and weight gradient) pointer is 16-byte aligned.
+int launch_gemm_f32(const GemmDesc& gr, const GemmDesc* gd, int epi, const float* row_scale, bool tables_aligned,
+                    hipStream_t st);
+int launch_xgemm_f32(const XGemm& g, int epi, bool tables_aligned, hipStream_t st);
+// K parts (1, 2, 4 or 8) of a dense fp32 weight gradient of groups x M x N outputs over k_len rows.
+int xgemm_f32_ksplit(int64_t M, int64_t N, int groups, int64_t k_len);
 // Few-row grouped GEMM (decode): row tiles of SK_BM rows, weights streamed
 // once.  The routed schedule must be built with bm = SK_BM; no G/U saves.
 constexpr int SK_BM = 64;
@@ -304,7 +313,7 @@ struct XGemm {
   int64_t gu_group_col;
   const float* row_w;
   int64_t du_off;
-  // XS_WGRAD split-K (MFMA path only): each group's K range is cut into
+  // XS_WGRAD split-K (MFMA kernels only): each group's K range is cut into
   // ksplit slab-aligned parts; part i writes fp32 partial sums to
   // part[((i * groups + grp) * M + m) * N + n] and a second kernel adds the
   // parts in ascending i and rounds once.  ksplit <= 1: direct store.
@@ -315,9 +324,9 @@ struct XGemm {
   int32_t c_f32;
 };
 
-// Backward grouped GEMM: MFMA kernel when dtype is bf16, allow_mfma is set
-// (the caller checked the alignment of every pointer-table entry) and the
-// shapes fit (xgemm_mfma_ok); fp32-FMA tiles otherwise.
+// Backward grouped GEMM.  fp32: gemm_f32.hip.  bf16: MFMA kernels when
+// allow_mfma is set (the caller checked the alignment of every pointer-table
+// entry) and the shapes fit (xgemm_q_ok, xgemm_mfma_ok); FMA tiles otherwise.
 int launch_xgemm(const XGemm& g, int epi, int dtype, bool allow_mfma, hipStream_t st);
 bool xgemm_mfma_ok(const XGemm& g, int epi);
 int launch_xgemm_mfma(const XGemm& g, int epi, hipStream_t st);

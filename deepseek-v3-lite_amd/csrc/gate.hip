@@ -13,7 +13,8 @@
 // work and the W traffic per workgroup shrink with ks.  With ks splits the
 // partial logits go to a workspace and the routing launch adds them in split
 // order; without a workspace (ks = 1) the workgroup routes its own tokens.
-// fp32 x: SIMT FMA tiles.
+// fp32 x in the layer: fp32 MFMA partial logits (gate_f32_kernel) and the same
+// routing launch.  Other shapes, and fp32 x without a workspace: SIMT FMA tiles.
 //
 // Routing.  One wave per token, one lane per expert (E <= 64; E <= 256 with
 // several experts per lane): sigmoid in double rounded once, + bias, then k
@@ -361,7 +362,78 @@ __global__ __launch_bounds__(RR_WAVES * 64) void route_rank_kernel(const float* 
   if (single) finish_single_block(sel, rank_lds, ntok, k, E, po, hist, off, til);
 }
 
-// ------------------------------------------------------------------ SIMT logits (fp32 x, or D % 64 != 0)
+// ------------------------------------------------------------------ fp32 MFMA logits (fp32 x)
+// A wave takes 32 tokens, every expert (NT tiles of 32) and one of ks ranges of
+// D / 8 column groups, and writes its partial logits; no LDS, no barrier.  Lane
+// half h of group g holds columns 8 g + 4 h .. + 3 of token (of x) and of expert
+// (of W) lane & 31, so one 16-byte load of each feeds four v_mfma_f32_32x32x2_f32.
+// Bound by latency: at T 2048, D 768, E 20 it reads 6.3 MB of x once, and W (61 KB)
+// from L2 for every token tile.  The FMA tiles it replaces in the layer put 128
+// tokens on a workgroup (16 workgroups at T 2048) and walked D in 32-column
+// chunks, one memory latency and two barriers each: 212 us there, 39 us at T 1024, D 64.
+constexpr int GF_TOK = 32;
+
+template <int NT>
+__global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__ x, const float* __restrict__ gw, int T,
+                                                       int D, int E, float* __restrict__ part, int ks,
+                                                       const PtrChunk tables, const void** tab_dst) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (blockIdx.x == 0)
+    for (int i = tid; i < tables.n; i += blockDim.x) tab_dst[tables.off + i] = tables.p[i];
+  const int64_t unit = (int64_t)blockIdx.x * 4 + (tid >> 6);   // (token tile, split), split fastest
+  const int split = (int)(unit % ks);
+  const int64_t t0 = unit / ks * GF_TOK;
+  if (t0 >= T) return;
+  const int groups = (D + 7) / 8, per = (groups + ks - 1) / ks;
+  const int g0 = split * per, g1 = min(groups, g0 + per);
+  const int m = lane & 31, kh = 4 * (lane >> 5);
+  const float* xr = x + min(t0 + m, (int64_t)T - 1) * D;
+  const float* wr[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) wr[i] = gw + (int64_t)min(32 * i + m, E - 1) * D;
+  g_f32x16_t acc[NT] = {};
+  constexpr int U = NT <= 2 ? 6 : NT <= 4 ? 4 : 2;   // groups in flight; groups past the range count as zeros
+  for (int g = g0; g < g1; g += U) {
+    g_f32x4_t xv[U], wv[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int kc = min(8 * (g + u) + kh, D - 4);   // D % 4 == 0: a half group is whole or absent
+      xv[u] = *reinterpret_cast<const g_f32x4_t*>(xr + kc);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) wv[u][i] = *reinterpret_cast<const g_f32x4_t*>(wr[i] + kc);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // keeps the batch's loads ahead of its MFMAs, all in flight
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = g + u < g1 && 8 * (g + u) + kh < D;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? wv[u][i][q] : 0.0f, in ? xv[u][q] : 0.0f, acc[i], 0, 0, 0);
+    }
+  }
+  // lane holds token m and, per q, experts 32 i + 8 q + 4 (lane >> 5) + {0..3}
+  if (t0 + m >= T) return;
+  float* pr = part + ((int64_t)split * T + t0 + m) * E;
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int e = 32 * i + 8 * q + kh;
+      if ((E & 3) == 0) {
+        if (e < E)
+          *reinterpret_cast<g_f32x4_t*>(pr + e) =
+              g_f32x4_t{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (e + r < E) pr[e + r] = acc[i][4 * q + r];
+      }
+    }
+}
+
+// ------------------------------------------------------------------ SIMT logits (other shapes)
 // LDS layout (floats): xs[KC][TB+4] | ws[KC][EC+4] | lg[TB][E+1] | bias[E] | hist[E] (int) | routing scratch
 // (64 ints per wave)
 template <typename XT, int EC>
@@ -542,6 +614,12 @@ static int gate_sc(const dsmoe_dims& d) {
 }
 
 int gate_k_splits(const dsmoe_dims& d) {
+  if (d.dtype == DSMOE_F32) {
+    // 32 columns or more per split, and no more splits than give each SIMD two waves
+    int ks = 1;
+    while (ks < GATE_KS_MAX && cdiv(d.T, GF_TOK) * ks * 2 <= 2048 && d.D >= 32 * ks * 2) ks *= 2;
+    return ks;
+  }
   const int64_t tiles = cdiv(d.T, GP_TOK);
   const int sc = gate_sc(d);
   int ks = 1;
@@ -557,13 +635,38 @@ static bool gate_mfma_ok(const void* x, const float* gw, const dsmoe_dims& d) {
          (reinterpret_cast<uintptr_t>(gw) & 15) == 0;
 }
 
-bool gate_uses_mfma(const void* x, const float* gw, const dsmoe_dims& d) { return d.T > 0 && gate_mfma_ok(x, gw, d); }
+// fp32 MFMA gate: 16-byte loads of x and W rows.
+static bool gate_f32_ok(const void* x, const float* gw, const dsmoe_dims& d) {
+  return d.dtype == DSMOE_F32 && d.D % 4 == 0 &&
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(gw)) & 15) == 0;
+}
+
+bool gate_uses_mfma(const void* x, const float* gw, const dsmoe_dims& d) {
+  return d.T > 0 && (gate_mfma_ok(x, gw, d) || gate_f32_ok(x, gw, d));
+}
+
+static int launch_gate_f32(const void* x, const float* gw, const float* bias, const dsmoe_dims& d, const GateOut& out,
+                           float* part, const PtrChunk* tables, const void** tab_dst, const PermuteOut* po,
+                           bool* ranked, hipStream_t st) {
+  PtrChunk none;
+  none.n = 0;
+  none.off = 0;
+  const int ks = gate_k_splits(d);
+  const unsigned blocks = (unsigned)cdiv(cdiv(d.T, GF_TOK) * ks, 4);
+  auto kern = d.E <= 32 ? gate_f32_kernel<1>
+              : d.E <= 64 ? gate_f32_kernel<2> : d.E <= 128 ? gate_f32_kernel<4> : gate_f32_kernel<8>;
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, st, static_cast<const float*>(x), gw, d.T, d.D, d.E, part, ks,
+                     tables ? *tables : none, tab_dst);
+  const int rc = check_launch("gate_f32");
+  if (rc) return rc;
+  return launch_route(part, ks, bias, d, out, po, ranked, st);
+}
 
 int launch_gate(const void* x, const float* logits_in, const float* gw, const float* bias, const dsmoe_dims& d,
                 const GateOut& out, hipStream_t st, float* part, const PtrChunk* tables, const void** tab_dst,
                 const PermuteOut* po, bool* ranked) {
   if (ranked) *ranked = false;
-  if (tables && (logits_in || !gate_uses_mfma(x, gw, d)))
+  if (tables && (logits_in || !part || !gate_uses_mfma(x, gw, d)))
     return fail(DSMOE_ERR_INVALID, "gate: a pointer table rides only with the MFMA gate");
   if (out.counts) {
     hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)cdiv(d.E, 256)), dim3(256), 0, st, out.counts, d.E, 0);
@@ -579,6 +682,7 @@ int launch_gate(const void* x, const float* logits_in, const float* gw, const fl
       default: return launch_gate_mfma_nt<8>(x, gw, bias, d, out, part, tables, tab_dst, po, ranked, st);
     }
   }
+  if (part && gate_f32_ok(x, gw, d)) return launch_gate_f32(x, gw, bias, d, out, part, tables, tab_dst, po, ranked, st);
   if (d.dtype == DSMOE_BF16) {
     if (d.E <= 16) return launch_gate_t<bf16_t, 16>(x, gw, bias, d, out, st);
     if (d.E <= 32) return launch_gate_t<bf16_t, 32>(x, gw, bias, d, out, st);

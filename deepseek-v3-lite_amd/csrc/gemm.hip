@@ -14,8 +14,9 @@
 // grid is sized from a host bound; blocks past the device count exit.
 //
 // Kernels (the default bf16 path is the persistent gemm_qp_kernel of
-// gemm_qp.hip; this file holds the register-staged MFMA kernel for the shapes
-// that one does not take, the fp32 fallback and the dispatcher):
+// gemm_qp.hip, the fp32 path gemm_f32.hip; this file holds the register-staged
+// MFMA kernel for the bf16 shapes that gemm_qp does not take, the FMA fallback
+// and the dispatcher):
 //   gemm_mfma_kernel  bf16 on gfx950 v_mfma_f32_32x32x16_bf16.  Block =
 //                     WM x WN waves, each owning TM x TN 32x32 output tiles
 //                     (x2 for SwiGLU: the W1 and W3 tiles of the same columns
@@ -24,8 +25,8 @@
 //                     buffered, XOR-swizzled 16-byte chunks) one slab ahead.
 //                     Rows past a tile's end are clamped to a valid row: their
 //                     results are discarded, so no load is predicated.
-//   gemm_simt_kernel  fp32 FMA fallback for fp32 and for shapes the MFMA
-//                     kernel does not take (any N, K, strides).
+//   gemm_simt_kernel  fp32 FMA fallback for bf16 shapes the MFMA kernels do
+//                     not take (any N, K, strides).
 #include <cstdlib>
 #include <cstring>
 
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const GemmDesc 
 constexpr int SM_N = 64;
 constexpr int SM_K = 16;
 
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const float* __restrict__ row_scale) {
   constexpr int NB = (EPI == EPI_SWIGLU) ? 2 : 1;
   __shared__ float As[SM_K][TILE_M + 4];
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const 
   const int n0 = n_tile * SM_N;
   const int tid = threadIdx.x;
   const int ty = tid >> 4, tx = tid & 15;  // rows ty*8.., cols tx*4..
-  const T* A = static_cast<const T*>(g.A);
+  const bf16_t* A = static_cast<const bf16_t*>(g.A);
   float acc[NB][8][4];
 #pragma unroll
   for (int b = 0; b < NB; ++b)
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const 
       float v = 0.0f;
       if (r < rows && k0 + kk < g.K) {
         const int64_t arow = g.a_map ? g.a_map[row0 + r] : (row0 + r);
-        v = to_f<T>(A[arow * g.lda + k0 + kk]);
+        v = bf2f(A[arow * g.lda + k0 + kk]);
       }
       As[kk][r] = v;
     }
@@ -258,8 +259,8 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const 
         float v = 0.0f;
         if (n0 + n < g.N && k < g.K) {
           const int seg = k / g.kseg;
-          const T* base = static_cast<const T*>((b == 0 ? g.B0 : g.B1)[grp * g.nseg + seg]);
-          v = to_f<T>(base[(int64_t)(n0 + n) * g.ldb + (k - seg * g.kseg)]);
+          const bf16_t* base = static_cast<const bf16_t*>((b == 0 ? g.B0 : g.B1)[grp * g.nseg + seg]);
+          v = bf2f(base[(int64_t)(n0 + n) * g.ldb + (k - seg * g.kseg)]);
         }
         Bs[b][kk][n] = v;
       }
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const 
     }
     __syncthreads();
   }
-  T* C = static_cast<T*>(g.C);
+  bf16_t* C = static_cast<bf16_t*>(g.C);
   const int64_t ccol = (int64_t)grp * g.c_group_col;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -298,11 +299,11 @@ __global__ __launch_bounds__(256) void gemm_simt_kernel(const GemmDesc g, const 
       const int64_t o = crow * g.ldc + ccol + n;
       if (EPI == EPI_SWIGLU) {
         const float gv = acc[0][i][j], uv = acc[NB - 1][i][j];
-        C[o] = from_f<T>(silu_f(gv) * uv);
-        if (g.Gs) static_cast<T*>(g.Gs)[o] = from_f<T>(gv);
-        if (g.Us) static_cast<T*>(g.Us)[o] = from_f<T>(uv);
+        C[o] = f2bf(silu_f(gv) * uv);
+        if (g.Gs) static_cast<bf16_t*>(g.Gs)[o] = f2bf(gv);
+        if (g.Us) static_cast<bf16_t*>(g.Us)[o] = f2bf(uv);
       } else {
-        C[o] = from_f<T>(acc[0][i][j] * scale);
+        C[o] = f2bf(acc[0][i][j] * scale);
       }
     }
   }
@@ -354,6 +355,7 @@ int launch_grouped_gemm(const GemmDesc& g_in, int epi, int dtype, const float* r
                         hipStream_t st) {
   const GemmDesc& g = g_in;
   if (g.N <= 0 || g.K <= 0) return DSMOE_OK;
+  if (dtype == DSMOE_F32) return launch_gemm_f32(g, nullptr, epi, row_scale, allow_mfma, st);
   if (gemm_mfma_eligible(g, dtype, allow_mfma)) {
     if (g.bm != MF_BM) return fail(DSMOE_ERR_INVALID, "gemm: schedule tile height does not match the MFMA kernel");
     if (gemm_qp_ok(g)) return launch_gemm_qp(g, epi, row_scale, st);
@@ -365,23 +367,18 @@ int launch_grouped_gemm(const GemmDesc& g_in, int epi, int dtype, const float* r
   if (g.bm != TILE_M) return fail(DSMOE_ERR_INVALID, "gemm: schedule tile height does not match the SIMT kernel");
   const int64_t grid = grid_for(g, TILE_M, SM_N);
   if (grid == 0) return DSMOE_OK;
-  if (dtype == DSMOE_BF16) {
-    if (epi == EPI_SWIGLU)
-      hipLaunchKernelGGL((gemm_simt_kernel<bf16_t, EPI_SWIGLU>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
-    else
-      hipLaunchKernelGGL((gemm_simt_kernel<bf16_t, EPI_STORE>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
-  } else {
-    if (epi == EPI_SWIGLU)
-      hipLaunchKernelGGL((gemm_simt_kernel<float, EPI_SWIGLU>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
-    else
-      hipLaunchKernelGGL((gemm_simt_kernel<float, EPI_STORE>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
-  }
+  if (epi == EPI_SWIGLU)
+    hipLaunchKernelGGL((gemm_simt_kernel<EPI_SWIGLU>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
+  else
+    hipLaunchKernelGGL((gemm_simt_kernel<EPI_STORE>), dim3((unsigned)grid), dim3(256), 0, st, g, row_scale);
   return check_launch("gemm_simt");
 }
 
 int launch_grouped_gemm_pair(const GemmDesc& gr_in, const GemmDesc& gd_in, int epi, int dtype, const float* row_scale,
                              bool allow_mfma_r, bool allow_mfma_d, hipStream_t st) {
   const GemmDesc &gr = gr_in, &gd = gd_in;
+  if (dtype == DSMOE_F32 && gd.sched == nullptr && gr.N > 0 && gr.K > 0 && gd.N > 0 && gd.K > 0)
+    return launch_gemm_f32(gr, &gd, epi, row_scale, allow_mfma_r && allow_mfma_d, st);
   const bool one = gd.sched == nullptr && gr.N > 0 && gr.K > 0 && gd.N > 0 &&
                    gd.K > 0 && gemm_mfma_eligible(gr, dtype, allow_mfma_r) && gemm_mfma_eligible(gd, dtype, allow_mfma_d) &&
                    gemm_qp_ok(gr) && gemm_qp_ok(gd);

@@ -12,7 +12,8 @@
 // each output tile is produced by one block that walks its K range in
 // ascending order, so dW accumulation is deterministic with no atomics.
 //
-// xgemm_simt_kernel: fp32 FMA tiles for every mode (fp32 path and fallback).
+// xgemm_simt_kernel: fp32 FMA tiles for every mode, for the bf16 shapes that
+// the MFMA kernels do not take.  fp32 runs gemm_f32.hip.
 #include "gemm_tile.h"
 
 namespace dsmoe {
@@ -21,34 +22,32 @@ constexpr int XS_BM = 64;
 constexpr int XS_BN = 64;
 constexpr int XS_BK = 16;
 
-template <typename T>
 __device__ __forceinline__ float xa_load(const XGemm& g, int grp, int row0, int m, int k) {
-  const T* A = static_cast<const T*>(g.A);
+  const bf16_t* A = static_cast<const bf16_t*>(g.A);
   if (g.a_mode == XA_ROWS) {
     const int r = row0 + m;
     const int64_t ar = g.a_map ? g.a_map[r] : r;
-    return to_f<T>(A[ar * g.lda + k]);
+    return bf2f(A[ar * g.lda + k]);
   }
   const int64_t ar = g.a_map ? g.a_map[k] : k;
   const float s = g.a_kscale ? g.a_kscale[k] : 1.0f;
-  return to_f<T>(A[ar * g.lda + (int64_t)grp * g.a_col + row0 + m]) * s;
+  return bf2f(A[ar * g.lda + (int64_t)grp * g.a_col + row0 + m]) * s;
 }
 
-template <typename T>
 __device__ __forceinline__ float xb_load(const XGemm& g, int grp, int n, int k) {
   if (g.b_mode == XB_ACT_KMAJOR) {
     const int64_t br = g.b_map ? g.b_map[k] : k;
-    return to_f<T>(static_cast<const T*>(g.Bact)[br * g.ldb + (int64_t)grp * g.b_col + n]);
+    return bf2f(static_cast<const bf16_t*>(g.Bact)[br * g.ldb + (int64_t)grp * g.b_col + n]);
   }
   const int seg = k / g.kseg;
   const int kin = k - seg * g.kseg;
-  const T* base = static_cast<const T*>(g.Btab[(int64_t)grp * g.nseg + seg]);
-  if (g.b_mode == XB_W_NT) return to_f<T>(base[(int64_t)n * g.ldb + kin]);
-  return to_f<T>(base[(int64_t)kin * g.ldb + n]);
+  const bf16_t* base = static_cast<const bf16_t*>(g.Btab[(int64_t)grp * g.nseg + seg]);
+  if (g.b_mode == XB_W_NT) return bf2f(base[(int64_t)n * g.ldb + kin]);
+  return bf2f(base[(int64_t)kin * g.ldb + n]);
 }
 
 // Shared epilogue for one output element (row m of the tile, column n).
-template <typename T, int EPI>
+template <int EPI>
 __device__ __forceinline__ void x_store(const XGemm& g, int grp, int row0, int m, int n, float acc) {
   if (EPI == XE_WGRAD) {
     const int mm = row0 + m;
@@ -57,28 +56,28 @@ __device__ __forceinline__ void x_store(const XGemm& g, int grp, int row0, int m
     if (g.c_f32)
       static_cast<float*>(base)[o] = acc;
     else
-      static_cast<T*>(base)[o] = from_f<T>(acc);
+      static_cast<bf16_t*>(base)[o] = f2bf(acc);
     return;
   }
   const int r = row0 + m;
   const int64_t crow = g.c_map ? g.c_map[r] : r;
-  T* C = static_cast<T*>(g.C);
+  bf16_t* C = static_cast<bf16_t*>(g.C);
   const int64_t o = crow * g.ldc + (int64_t)grp * g.c_group_col + n;
   if (EPI == XE_STORE) {
-    C[o] = from_f<T>(acc);
+    C[o] = f2bf(acc);
     return;
   }
   // SwiGLU backward: h = silu(gv) * uv, dh = w * acc
   const int64_t ogu = (int64_t)r * g.ld_gu + (int64_t)grp * g.gu_group_col + n;
-  const float gv = to_f<T>(static_cast<const T*>(g.Gs)[ogu]);
-  const float uv = to_f<T>(static_cast<const T*>(g.Us)[ogu]);
+  const float gv = bf2f(static_cast<const bf16_t*>(g.Gs)[ogu]);
+  const float uv = bf2f(static_cast<const bf16_t*>(g.Us)[ogu]);
   const float dh = (g.row_w ? g.row_w[r] : 1.0f) * acc;
   const float sg = sigmoid_f(gv);
-  C[o] = from_f<T>(dh * uv * sg * (1.0f + gv * (1.0f - sg)));
-  C[o + g.du_off] = from_f<T>(dh * gv * sg);
+  C[o] = f2bf(dh * uv * sg * (1.0f + gv * (1.0f - sg)));
+  C[o + g.du_off] = f2bf(dh * gv * sg);
 }
 
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void xgemm_simt_kernel(const XGemm g) {
   __shared__ float As[XS_BK][XS_BM + 4];
   __shared__ float Bs[XS_BK][XS_BN + 4];
@@ -100,7 +99,7 @@ __global__ __launch_bounds__(256) void xgemm_simt_kernel(const XGemm g) {
         kk = i - m * XS_BK;
       }
       float v = 0.0f;
-      if (m < rows && k0 + kk < kend) v = xa_load<T>(g, grp, row0, m, k0 + kk);
+      if (m < rows && k0 + kk < kend) v = xa_load(g, grp, row0, m, k0 + kk);
       As[kk][m] = v;
     }
     for (int i = tid; i < XS_BN * XS_BK; i += 256) {
@@ -113,7 +112,7 @@ __global__ __launch_bounds__(256) void xgemm_simt_kernel(const XGemm g) {
         n = i - kk * XS_BN;
       }
       float v = 0.0f;
-      if (n0 + n < g.N && k0 + kk < kend) v = xb_load<T>(g, grp, n0 + n, k0 + kk);
+      if (n0 + n < g.N && k0 + kk < kend) v = xb_load(g, grp, n0 + n, k0 + kk);
       Bs[kk][n] = v;
     }
     __syncthreads();
@@ -138,7 +137,7 @@ __global__ __launch_bounds__(256) void xgemm_simt_kernel(const XGemm g) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + tx * 4 + j;
-      if (n < g.N) x_store<T, EPI>(g, grp, row0, m, n, acc[i][j]);
+      if (n < g.N) x_store<EPI>(g, grp, row0, m, n, acc[i][j]);
     }
   }
 }
@@ -154,23 +153,23 @@ static int64_t xgrid(const XGemm& g, int bm, int bn) {
   return 8 * cdiv(m_bound * cdiv(g.N, bn), 8);
 }
 
-template <typename T>
 static int launch_xsimt(const XGemm& g, int epi, hipStream_t st) {
   const int64_t grid = xgrid(g, XS_BM, XS_BN);
   if (grid == 0) return DSMOE_OK;
   if (epi == XE_STORE)
-    hipLaunchKernelGGL((xgemm_simt_kernel<T, XE_STORE>), dim3((unsigned)grid), dim3(256), 0, st, g);
+    hipLaunchKernelGGL((xgemm_simt_kernel<XE_STORE>), dim3((unsigned)grid), dim3(256), 0, st, g);
   else if (epi == XE_SWIGLU_BWD)
-    hipLaunchKernelGGL((xgemm_simt_kernel<T, XE_SWIGLU_BWD>), dim3((unsigned)grid), dim3(256), 0, st, g);
+    hipLaunchKernelGGL((xgemm_simt_kernel<XE_SWIGLU_BWD>), dim3((unsigned)grid), dim3(256), 0, st, g);
   else
-    hipLaunchKernelGGL((xgemm_simt_kernel<T, XE_WGRAD>), dim3((unsigned)grid), dim3(256), 0, st, g);
+    hipLaunchKernelGGL((xgemm_simt_kernel<XE_WGRAD>), dim3((unsigned)grid), dim3(256), 0, st, g);
   return check_launch("xgemm_simt");
 }
 
 int launch_xgemm(const XGemm& g, int epi, int dtype, bool allow_mfma, hipStream_t st) {
   if (g.N <= 0 || (g.sched_mode == XS_WGRAD ? g.M <= 0 : false)) return DSMOE_OK;
-  if (dtype == DSMOE_BF16 && allow_mfma && xgemm_q_ok(g, epi)) return launch_xgemm_q(g, epi, st);
-  if (dtype == DSMOE_BF16 && allow_mfma && xgemm_mfma_ok(g, epi)) return launch_xgemm_mfma(g, epi, st);
+  if (dtype == DSMOE_F32) return launch_xgemm_f32(g, epi, allow_mfma, st);
+  if (allow_mfma && xgemm_q_ok(g, epi)) return launch_xgemm_q(g, epi, st);
+  if (allow_mfma && xgemm_mfma_ok(g, epi)) return launch_xgemm_mfma(g, epi, st);
   if (g.ksplit > 1) {  // the FMA tiles store directly
     XGemm g1 = g;
     g1.ksplit = 1;
@@ -178,8 +177,7 @@ int launch_xgemm(const XGemm& g, int epi, int dtype, bool allow_mfma, hipStream_
   }
   if (g.sched_mode == XS_ROUTED && g.bm % XS_BM != 0)
     return fail(DSMOE_ERR_INVALID, "xgemm: schedule height must be a multiple of 64");
-  if (dtype == DSMOE_BF16) return launch_xsimt<bf16_t>(g, epi, st);
-  return launch_xsimt<float>(g, epi, st);
+  return launch_xsimt(g, epi, st);
 }
 
 }  // namespace dsmoe
