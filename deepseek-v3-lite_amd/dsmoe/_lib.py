@@ -46,6 +46,7 @@ P = ctypes.c_void_p
 PP = ctypes.POINTER(ctypes.c_void_p)
 DIMS = ctypes.POINTER(Dims)
 I32 = ctypes.c_int
+I64 = ctypes.c_int64
 F32 = ctypes.c_float
 SZ = ctypes.c_size_t
 
@@ -76,6 +77,8 @@ _SIGNATURES = {
     "dsmoe_mla_attn_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),
     "dsmoe_mla_attn_fwd": ([P, P, P, P, P, P, ctypes.POINTER(MlaDims), P, P, SZ, P], I32),
     "dsmoe_mla_attn_fwd_lse": ([P, P, P, P, P, P, ctypes.POINTER(MlaDims), P, P, P, SZ, P], I32),
+    "dsmoe_mla_attn_few_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),
+    "dsmoe_mla_attn_few": ([P, P, P, P, P, I64, P, I64, ctypes.POINTER(MlaDims), P, P, P, SZ, P], I32),
     "dsmoe_mla_attn_bwd_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),
     "dsmoe_mla_attn_kv": ([P, P, P, P, ctypes.POINTER(MlaDims), P, SZ, P], I32),
     "dsmoe_mla_attn_bwd": ([P, P, ctypes.POINTER(MlaDims), P, SZ, P, P, P, P, P, P, P, P, SZ, P], I32),

@@ -31,8 +31,8 @@ CFLAGS = [
 ]
 # Per-source flags: the attention kernels keep MFMA accumulators in VGPRs (their
 # online-softmax rescaling reads and writes them every key block).
-EXTRA_FLAGS = {"mla.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-SOURCES = ["api.hip", "gate.hip", "permute.hip", "gemm.hip", "gemm_f32.hip", "gemm_qp.hip", "gemm_sk.hip", "gemm_x.hip", "gemm_xm.hip", "gemm_xq.hip", "bwd.hip", "combine.hip", "mla.hip"]
+EXTRA_FLAGS = {"mla.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "mla_few.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+SOURCES = ["api.hip", "gate.hip", "permute.hip", "gemm.hip", "gemm_f32.hip", "gemm_qp.hip", "gemm_sk.hip", "gemm_x.hip", "gemm_xm.hip", "gemm_xq.hip", "bwd.hip", "combine.hip", "mla.hip", "mla_few.hip"]
 PROBE_SOURCES = ["probe.hip"]
 
 

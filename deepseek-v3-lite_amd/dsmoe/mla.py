@@ -99,13 +99,57 @@ def _prepare(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v):
         raise ValueError(f"mla_attention: H * S_kv = {H * S_kv} (H * S_q = {H * S_q}) reaches 2^22, the limit of "
                          "one batch row of the kernels' 32-bit row offsets")
     bc = min(B, (_ROWS_PER_CALL - 1) // per_batch)
+    if _few(S_q, R, D_nope, D_v) and _head_rows(wkv_b_k) and _head_rows(wkv_b_v):
+        return (*(t.contiguous() for t in ts[:4]), wkv_b_k, wkv_b_v), bc
     return tuple(t.contiguous() for t in ts), bc
+
+
+def _few(S_q: int, R: int, D_nope: int, D_v: int) -> bool:
+    """Whether the attention of S_q queries runs on the latent rows
+    (csrc/mla_few.hip) instead of building K and V: where that takes fewer
+    multiplications, 3 R + D_rope for each (query, key) against
+    2 D_nope + D_rope + D_v and R (D_nope + D_v) for each key, and no more than 32
+    queries (measured at the 422m widths, S_kv 1537: 55 against 74 us at B 8 and
+    26 against 49 at B 1 with 32 queries; from 128 to 256 queries the K and V
+    path is the faster one)."""
+    return S_q <= 32 and S_q * (3 * R - 2 * D_nope - D_v) <= R * (D_nope + D_v)
+
+
+def _head_rows(w: torch.Tensor) -> bool:
+    """(H, D, R) weights whose heads are D contiguous rows each, at any distance
+    from one another: the per-head views of wkv_b.weight as well as whole tensors."""
+    return w.stride(2) == 1 and w.stride(1) == w.size(2)
+
+
+def _forward_few(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int):
+    """dsmoe_mla_attn_few over the batch chunks: bf16 out and the fp32 lse."""
+    q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v = ts
+    B, H, S_q, _ = q_nope.shape
+    dev = q_nope.device
+    lib = L.load()
+    d = _dims(q_nope[:bc], q_pe, ctx_kv, wkv_b_v, softmax_scale, is_causal, q_start)
+    nbytes = int(lib.dsmoe_mla_attn_few_workspace_size(d))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    out = torch.empty(B, S_q, H, wkv_b_v.size(1), dtype=torch.bfloat16, device=dev)
+    lse = torch.empty(B, H, S_q, dtype=torch.float32, device=dev)
+    for b0 in range(0, B, bc):
+        b1 = min(B, b0 + bc)
+        c = (q_nope, q_pe, ctx_kv, ctx_pe, out, lse)
+        if bc < B:
+            c = tuple(t[b0:b1] for t in c)
+            d.B = b1 - b0
+        L.check(lib.dsmoe_mla_attn_few(L.ptr(c[0]), L.ptr(c[1]), L.ptr(c[2]), L.ptr(c[3]), L.ptr(wkv_b_k),
+                                       wkv_b_k.stride(0), L.ptr(wkv_b_v), wkv_b_v.stride(0), d, L.ptr(c[4]),
+                                       L.ptr(c[5]), L.ptr(ws), nbytes, L.stream_ptr(dev)), "dsmoe_mla_attn_few")
+    return out, lse
 
 
 def _forward(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int, want_lse: bool):
     """dsmoe_mla_attn_fwd (or _fwd_lse) over the batch chunks: bf16 out, the
     fp32 lse (None unless asked for) and the workspace, which holds the last
-    chunk's K and V."""
+    chunk's K and V; None for a few queries, whose attention builds neither."""
+    if _few(ts[0].size(2), ts[2].size(2), ts[0].size(3), ts[5].size(1)):
+        return (*_forward_few(ts, bc, softmax_scale, is_causal, q_start), None)
     q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v = ts
     B, H, S_q, _ = q_nope.shape
     D_v = wkv_b_v.size(1)
@@ -156,6 +200,7 @@ def mla_attention_bwd_heads(ts, bc: int, out: torch.Tensor, lse: torch.Tensor, d
     B, H, S_q, Dn = q_nope.shape
     S_kv, Dr, Dv = ctx_kv.size(1), q_pe.size(-1), wkv_b_v.size(1)
     dev = q_nope.device
+    wkv_b_k, wkv_b_v = wkv_b_k.contiguous(), wkv_b_v.contiguous()
     dout = dout.to(torch.bfloat16).contiguous()
     lib = L.load()
     d = _dims(q_nope[:bc], q_pe[:bc], ctx_kv[:bc], wkv_b_v, softmax_scale, is_causal, q_start)
@@ -220,7 +265,7 @@ class _MlaAttentionFunction(torch.autograd.Function):
         # forward's K and V when one launch covered the batch (B H pad64(S_kv)
         # (DQKp + DVp) bf16, held until the backward); otherwise it rebuilds them
         ctx.save_for_backward(*ts, out, lse)
-        ctx.kv_ws = kv_ws if bc >= ts[0].size(0) else None
+        ctx.kv_ws = kv_ws if bc >= ts[0].size(0) else None   # (None too after a few queries)
         ctx.args = (bc, softmax_scale, is_causal, q_start)
         return out if out_dtype == torch.bfloat16 else out.to(out_dtype)
 

@@ -291,6 +291,21 @@ int dsmoe_mla_attn_fwd(const void* q_nope, const void* q_pe, const void* ctx_kv,
 int dsmoe_mla_attn_fwd_lse(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
                            const void* wkv_b_k, const void* wkv_b_v, const dsmoe_mla_dims* dims, void* out,
                            float* lse, void* workspace, size_t workspace_bytes, void* stream);
+/* The same attention for a few queries over a long cache (decoding): the query
+ * is taken to the latent rows (q_nope W_k . ctx_kv) and the attention runs on
+ * them, so no K and V are built; ranges of keys run side by side and are added
+ * at the end.  No counterpart in the reference.  lse may be NULL, else as
+ * dsmoe_mla_attn_fwd_lse writes it (a backward needs kv_ws from
+ * dsmoe_mla_attn_kv).  The up-projections of a head are D_nope (D_v) rows of R
+ * contiguous elements; consecutive heads' are wk_head_stride (wv_head_stride)
+ * elements apart, so the per-head views of one wkv_b weight are read in place.
+ * The workspace holds the taken queries and the ranges' partial sums
+ * (dsmoe_mla_attn_few_workspace_size; 0 for dims no attention call takes). */
+size_t dsmoe_mla_attn_few_workspace_size(const dsmoe_mla_dims* dims);
+int dsmoe_mla_attn_few(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
+                       const void* wkv_b_k, int64_t wk_head_stride, const void* wkv_b_v, int64_t wv_head_stride,
+                       const dsmoe_mla_dims* dims, void* out, float* lse, void* workspace, size_t workspace_bytes,
+                       void* stream);
 /* K and V of every (batch, head) into kv_ws (dsmoe_mla_attn_workspace_size
  * bytes), the first launch of dsmoe_mla_attn_fwd on its own: for a backward
  * whose caller did not keep the forward's workspace.  No counterpart in the

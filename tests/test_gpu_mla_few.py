@@ -1,0 +1,82 @@
+"""GPU parity of the attention of a few queries on the latent rows (csrc/mla_few.hip) against the float64 oracle,
+with the bar of tests/test_gpu_mla.py, at the edges of its tiles, key ranges and load forms."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.mla_ref import mla_attention_oracle
+from tests.test_gpu_mla import ATOL, DEV, RTOL, _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(ts, sc, causal, q_start):
+    import dsmoe.mla as M
+    assert M._few(ts[0].size(2), ts[2].size(2), ts[0].size(3), ts[5].size(1)), "not the path under test"
+    out = M.mla_attention(*ts, sc, is_causal=causal, q_start=q_start)
+    torch.cuda.synchronize()
+    return out
+
+
+def _check(out, ts, sc, causal, q_start):
+    ref = mla_attention_oracle(*[t.detach().cpu() for t in ts], sc, is_causal=causal, q_start=q_start)
+    got = out.detach().float().cpu().numpy().astype(np.float64)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - ref) <= ATOL + RTOL * np.abs(ref)).all(), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("B,H,S_q,S_kv,R,Dn,Dr,Dv,causal,q_start", [
+    (1, 1, 1, 1, 192, 48, 24, 64, True, 0),            # one key
+    (2, 12, 1, 33, 192, 48, 24, 64, True, 32),         # a second chunk of one key
+    (2, 12, 1, 100, 192, 48, 24, 64, True, 40),        # keys past the query's position stay masked, ranges without keys
+    (1, 12, 32, 300, 192, 48, 24, 64, True, 268),      # the most queries, several row tiles
+    (3, 5, 7, 129, 128, 64, 32, 48, True, 60),         # a row tile over several queries
+    (1, 40, 1, 5000, 256, 128, 64, 128, False, 0),     # two row tiles, several chunks per range, no mask
+    (2, 3, 2, 70, 20, 10, 6, 12, True, 5),             # element loads
+    (1, 2, 4, 65, 8, 16, 8, 16, True, 61),             # a latent row of one 16-byte chunk
+    (40, 4, 1, 600, 16, 16, 16, 16, True, 599),
+    (1, 2, 1, 8200, 64, 32, 16, 32, True, 8199),       # as many ranges as there may be
+])
+def test_few_queries(B, H, S_q, S_kv, R, Dn, Dr, Dv, causal, q_start):
+    ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=S_kv)
+    _check(_run(ts, sc, causal, q_start), ts, sc, causal, q_start)
+
+
+@pytest.mark.parametrize("scale", [-0.3, 2.0])
+def test_scales(scale):
+    ts, _ = _inputs(1, 4, 2, 200, 64, 32, 16, 32, seed=3)
+    _check(_run(ts, scale, True, 150), ts, scale, True, 150)
+
+
+def test_head_views_and_unaligned_rows():
+    """The per-head views of one weight, and latent rows two bytes past a 16-byte boundary: the aligned call's
+    result, bit for bit (the same values in the same order)."""
+    B, H, S_q, S_kv, R, Dn, Dr, Dv = 2, 3, 1, 90, 64, 32, 16, 24
+    ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=4)
+    w = torch.cat([ts[4], ts[5]], 1).reshape(H * (Dn + Dv), R).view(H, Dn + Dv, R)
+    shifted = torch.empty(ts[2].numel() + 1, dtype=torch.bfloat16, device=DEV)[1:].view(ts[2].shape)
+    shifted.copy_(ts[2])
+    a = _run(ts, sc, True, 89)
+    b = _run((*ts[:4], w[:, :Dn], w[:, Dn:]), sc, True, 89)
+    c = _run((ts[0], ts[1], shifted, *ts[3:]), sc, True, 89)
+    assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def test_gradients():
+    """The backward builds K and V itself; it takes the log-sum-exp of this forward."""
+    B, H, S_q, S_kv, R, Dn, Dr, Dv = 2, 3, 3, 70, 32, 16, 8, 24
+    ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=5, wscale=0.3)
+    w = torch.cat([ts[4], ts[5]], 1).requires_grad_()
+    ins = [t.clone().requires_grad_() for t in ts[:4]]
+    out = _run((*ins, w[:, :Dn], w[:, Dn:]), sc, True, 60)
+    dout = torch.randn_like(out)
+    out.backward(dout)
+    qn, qp, kv, pe, w64 = [t.detach().double().requires_grad_() for t in (*ts[:4], w)]
+    k = torch.cat([torch.einsum("bsr,hdr->bhsd", kv, w64[:, :Dn]), pe[:, None].expand(B, H, S_kv, Dr)], -1)
+    v = torch.einsum("bsr,hdr->bhsd", kv, w64[:, Dn:])
+    z = torch.cat([qn, qp], -1) @ k.transpose(2, 3) * sc
+    mask = torch.arange(S_kv, device=DEV)[None] > torch.arange(S_q, device=DEV)[:, None] + 60
+    o = z.masked_fill(mask, float("-inf")).softmax(-1) @ v
+    o.transpose(1, 2).backward(dout.double())
+    for a, b in zip((*ins, w), (qn, qp, kv, pe, w64)):
+        assert (a.grad.double() - b.grad).abs().max() <= 2e-2 + 2e-2 * b.grad.abs().max()
