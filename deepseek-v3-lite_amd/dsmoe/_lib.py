@@ -85,6 +85,26 @@ _SIGNATURES = {
 }
 
 _lib = None
+_layer_fns = None
+
+
+def layer_fns():
+    """(host module, dsmoe_moe_fwd, dsmoe_moe_bwd_ex) of the eager layer path: the
+    two functions take their host pointer arrays as bytes (the host module's)."""
+    global _layer_fns
+    if _layer_fns is None:
+        lib = load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise ImportError(f"dsmoe: {LIB_PATH.parent / '_host.so'} is not built or does not load ({e}); run "
+                              "__graft_entry__.build() (or `python -m dsmoe.build` in deepseek-v3-lite_amd/)") from e
+        fns = []
+        for name in ("dsmoe_moe_fwd", "dsmoe_moe_bwd_ex"):
+            args, res = _SIGNATURES[name]
+            fns.append(ctypes.CFUNCTYPE(res, *[P if a is PP else a for a in args])((name, lib)))
+        _layer_fns = (_host, *fns)
+    return _layer_fns
 
 
 def load() -> ctypes.CDLL:
@@ -126,7 +146,7 @@ def dtype_code(dtype: torch.dtype) -> int:
 
 def ptr(t):
     """Device pointer of a tensor (None -> NULL)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def ptr_array(ts: Iterable[torch.Tensor]):
@@ -135,8 +155,18 @@ def ptr_array(ts: Iterable[torch.Tensor]):
     return ctypes.cast(arr, PP), arr  # keep `arr` alive while the call runs
 
 
+def stack_array(t: torch.Tensor):
+    """Host array of the device pointers of t[0], t[1], ... (t contiguous)."""
+    n, p = t.size(0), t.data_ptr()
+    step = t.stride(0) * t.element_size()
+    arr = (ctypes.c_void_p * max(n, 1))(*[p + i * step for i in range(n)])
+    return ctypes.cast(arr, PP), arr  # keep `arr` alive while the call runs
+
+
 def stream_ptr(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """hipStream_t of the device's current stream."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def timing_enable(on: bool) -> None:

@@ -1,4 +1,5 @@
-"""Compile the HIP sources in ../csrc into dsmoe/libdsmoe.so for gfx950.
+"""Compile the HIP sources in ../csrc into dsmoe/libdsmoe.so for gfx950, and
+../csrc/host.cpp (host code over the CPython and torch C++ APIs) into dsmoe/_host.so.
 
 Run as ``python -m dsmoe.build`` (from deepseek-v3-lite_amd/) or through
 ``__graft_entry__.build()``.  hipcc cross-compiles without a GPU.
@@ -19,6 +20,7 @@ CSRC = ROOT / "csrc"
 INCLUDE = REPO / "include"
 BUILD = ROOT / "_build"
 LIB = PKG / "libdsmoe.so"
+HOST_LIB = PKG / "_host.so"               # per-tensor host work of a layer call
 PROBE_LIB = PKG / "libdsmoe_probe.so"     # measurement tooling (bench.py --dma-mb), not the layer
 
 ARCH = "gfx950"
@@ -48,6 +50,24 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _compile_host() -> None:
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    tmp = HOST_LIB.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{p}" for p in (*include_paths(), sysconfig.get_paths()["include"])], str(CSRC / "host.cpp"),
+           "-o", str(tmp), *[f"-L{p}" for p in library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{r.stdout}\n{r.stderr}")
+    if r.stderr.strip():
+        print(f"[dsmoe.build] host.cpp:\n{r.stderr}", file=sys.stderr)
+    tmp.replace(HOST_LIB)
+
+
 def _link(objs, out: Path) -> None:
     tmp = out.with_suffix(".so.tmp")
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
@@ -58,12 +78,14 @@ def _link(objs, out: Path) -> None:
 
 
 def build(verbose: bool = True) -> Path:
-    """Compile every source and link libdsmoe.so and the measurement probe
-    library libdsmoe_probe.so (always rebuilds)."""
+    """Compile every source and link libdsmoe.so, the host module _host.so and
+    the measurement probe library libdsmoe_probe.so (always rebuilds)."""
     BUILD.mkdir(exist_ok=True)
     srcs = [CSRC / s for s in SOURCES + PROBE_SOURCES]
     with ThreadPoolExecutor(max_workers=min(len(srcs), 8)) as ex:
+        host = ex.submit(_compile_host)
         objs = list(ex.map(_compile, srcs))
+        host.result()
     _link(objs[:len(SOURCES)], LIB)
     _link(objs[len(SOURCES):], PROBE_LIB)
     if verbose:

@@ -196,6 +196,14 @@ class DeepSeekMoE(nn.Module):
 
     def _expert_params(self):
         """Expert weight parameters in the layer operator's order."""
+        if not torch.compiler.is_compiling():
+            # the modules' own tables: attribute access through nn.Module costs
+            # about 1 us for each of the 3 (E + S) weights
+            try:
+                groups = [list(m._modules.values()) for m in (self.experts, self.shared_experts)]
+                return [e._modules[n]._parameters["weight"] for es in groups for n in ("w1", "w2", "w3") for e in es]
+            except (AttributeError, KeyError):
+                pass   # parametrised weights, other expert modules
         return ([e.w1.weight for e in self.experts] + [e.w2.weight for e in self.experts] +
                 [e.w3.weight for e in self.experts] + [e.w1.weight for e in self.shared_experts] +
                 [e.w2.weight for e in self.shared_experts] + [e.w3.weight for e in self.shared_experts])
@@ -204,17 +212,6 @@ class DeepSeekMoE(nn.Module):
         # .to() / .cuda() / .half() replace parameter data: drop the cast copies
         self._cast_cache.clear()
         return super()._apply(fn, *args, **kwargs)
-
-    def _expert_weights(self, dtype: torch.dtype):
-        def cast(w):
-            return self._cast(w, dtype)
-        w1 = [cast(e.w1.weight) for e in self.experts]
-        w2 = [cast(e.w2.weight) for e in self.experts]
-        w3 = [cast(e.w3.weight) for e in self.experts]
-        s1 = [cast(e.w1.weight) for e in self.shared_experts]
-        s2 = [cast(e.w2.weight) for e in self.shared_experts]
-        s3 = [cast(e.w3.weight) for e in self.shared_experts]
-        return w1, w2, w3, s1, s2, s3
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """Flatten -> fused gate -> permute -> grouped SwiGLU -> combine + shared."""
@@ -231,12 +228,10 @@ class DeepSeekMoE(nn.Module):
             # bf16 copies and the backward writes fp32 gradients for the
             # parameters themselves (no per-parameter cast nodes)
             masters = params
-            copies = [self._cached_copy(p, cdt) for p in params]
-            E, S = self.n_routed_experts, self.n_shared_experts
-            w1, w2, w3 = copies[:E], copies[E:2 * E], copies[2 * E:3 * E]
-            s1, s2, s3 = copies[3 * E:3 * E + S], copies[3 * E + S:3 * E + 2 * S], copies[3 * E + 2 * S:]
+            weights = [self._cached_copy(p, cdt) for p in params]
         else:
-            w1, w2, w3, s1, s2, s3 = self._expert_weights(cdt)
+            weights = [p if p.dtype == cdt else self._cast(p, cdt) for p in params]
+        w1, w2, w3, s1, s2, s3 = ops._layer_weights(weights, len(self.experts), len(self.shared_experts))
         y, idx64, wx, counts = ops.moe_layer(flat.to(cdt), _flt(self.gate.weight), _flt(self.gate.bias), w1, w2, w3,
                                              s1, s2, s3, k=self.gate.topk, route_scale=self.gate.route_scale,
                                              master_weights=masters)

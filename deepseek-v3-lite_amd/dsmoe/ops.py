@@ -13,6 +13,7 @@ from __future__ import annotations
 from typing import List, Optional, Sequence, Tuple
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib as L
 
@@ -277,6 +278,107 @@ def _moe_fwd_backward(ctx, dy, _didx, _dwx, _dcounts, _dws):
 torch.library.register_autograd("dsmoe::moe_fwd", _moe_fwd_backward, setup_context=_moe_fwd_setup)
 
 
+# ---------------------------------------------------------------------------- eager layer
+# A torch.library operator with 3 (E + S) weights in a list costs 0.08 ms per
+# call without autograd and 1.1 ms with it (E 64, S 2: schema conversion, pytree
+# flattening and per-tensor checks in Python), several times the kernels of a
+# decode step.  A plain eager call therefore runs the same two C functions
+# through an ordinary autograd function; whatever looks at operators (a compiler
+# or tracer, a dispatch or function mode, a functional transform, forward-mode
+# AD, tensor subclasses) gets the operator.
+def _plain_eager() -> bool:
+    return not (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+                or torch._C._len_torch_function_stack() or torch._C._get_tracing_state() is not None
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0)
+
+
+def _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, route_scale, training):
+    """dsmoe_moe_fwd on checked tensors: (y, idx64, weights_x, counts int32, workspace u8)."""
+    dev = x.device
+    T, D = x.shape
+    d = L.make_dims(T, D, E, k, I, S, I_s, x.dtype, route_scale)
+    ws = _ws(L.load().dsmoe_moe_fwd_workspace_size(d, int(training)), dev)
+    y = torch.empty_like(x)
+    idx64 = torch.empty(T, k, dtype=torch.int64, device=dev)
+    wx = torch.empty(T, k, dtype=x.dtype, device=dev)
+    counts = torch.empty(E, dtype=torch.int32, device=dev)
+    rc = L.layer_fns()[1](x.data_ptr(), gate_w.data_ptr(), gate_bias.data_ptr(), *arrays, d, int(training),
+                          y.data_ptr(), idx64.data_ptr(), wx.data_ptr(), counts.data_ptr(), None, ws.data_ptr(),
+                          ws.numel(), L.stream_ptr(dev))
+    L.check(rc, "dsmoe_moe_fwd")
+    return y, idx64, wx, counts, ws
+
+
+class _LayerFn(torch.autograd.Function):
+    """The eager layer under autograd: as dsmoe::moe_fwd / dsmoe::moe_bwd."""
+
+    @staticmethod
+    def forward(ctx, meta, arrays, x, gate_w, gate_bias, *tensors):
+        E, S, k, I, I_s, rs, training = meta
+        n = 3 * (E + S)
+        y, idx64, wx, counts, ws = _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, rs, training)
+        ctx.meta = (*meta, len(tensors) - n)
+        ctx.save_for_backward(x, gate_w, ws, *tensors[:n])
+        ctx.set_materialize_grads(False)   # only y carries a gradient
+        return y, idx64, wx, counts
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dy, _didx, _dwx, _dcounts):
+        E, S, k, I, I_s, rs, training, n_masters = ctx.meta
+        x, gate_w, ws, *weights = ctx.saved_tensors
+        n = len(weights)
+        if dy is None:
+            return (None,) * (5 + n + n_masters)
+        if not training:
+            raise RuntimeError("dsmoe: forward ran without saving activations for backward")
+        dy = _c(dy)
+        host, _, bwd = L.layer_fns()
+        # a saved-tensor hook may hand back tensors of another kind or place than it
+        # was given; those go through the operator, as do the observers' calls
+        found = host.scan(weights, [], x, gate_w, None, E, S, k) if _plain_eager() else None
+        if found is None or found[:2] != (I, I_s) or ws.device != x.device or not ws.is_contiguous():
+            g = moe_bwd_op(x, gate_w, weights, dy, ws, E, S, k, I, I_s, rs, n_masters > 0)
+            dx, dgw, dws = g[0], g[1], g[2:]
+        else:
+            dev = x.device
+            T, D = x.shape
+            d = L.make_dims(T, D, E, k, I, S, I_s, x.dtype, rs)
+            bws = _ws(L.load().dsmoe_moe_bwd_workspace_size(d), dev)
+            dx = torch.empty_like(x)
+            dgw = torch.empty(E, D, dtype=torch.float32, device=dev)
+            if n_masters:
+                dws = [torch.empty_like(w, dtype=torch.float32) for w in weights]
+            else:
+                dws = [torch.empty_like(w) for w in weights]
+            rc = bwd(x.data_ptr(), gate_w.data_ptr(), *found[3], d, dy.data_ptr(), ws.data_ptr(), dx.data_ptr(),
+                     dgw.data_ptr(), *[host.addresses(a) for a in _layer_weights(dws, E, S)],
+                     L.DSMOE_F32 if n_masters else L.dtype_code(x.dtype), bws.data_ptr(), bws.numel(),
+                     L.stream_ptr(dev))
+            L.check(rc, "dsmoe_moe_bwd_ex")
+        if n_masters:
+            return (None, None, dx, dgw, None, *([None] * n), *dws)
+        return (None, None, dx, dgw, None, *dws)
+
+
+def _eager_layer(x, gate_w, gate_bias, weights, masters, E, S, k, route_scale, training):
+    """The layer of a plain eager call: (y, idx64, weights_x, counts), or None
+    when the call is not one (the operator path then checks and runs it)."""
+    if not _plain_eager():
+        return None
+    found = L.layer_fns()[0].scan(weights, masters, x, gate_w, gate_bias, E, S, k)
+    if found is None:
+        return None
+    I, I_s, needs_grad, arrays = found
+    grad = torch.is_grad_enabled() and needs_grad
+    if training is None:
+        training = grad
+    if not grad:
+        return _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, route_scale, training)[:4]
+    return _LayerFn.apply((E, S, k, I, I_s, route_scale, bool(training)), arrays, x, gate_w, gate_bias, *weights, *masters)
+
+
 def check_layer_args(x: torch.Tensor, gate_w: torch.Tensor, gate_bias: torch.Tensor, w1: Sequence[torch.Tensor],
                      w2: Sequence[torch.Tensor], w3: Sequence[torch.Tensor], sw1: Sequence[torch.Tensor],
                      sw2: Sequence[torch.Tensor], sw3: Sequence[torch.Tensor], k: int) -> Tuple[int, int, int, int]:
@@ -335,6 +437,12 @@ def moe_layer(x: torch.Tensor, gate_w: torch.Tensor, gate_bias: torch.Tensor, w1
     are bf16 copies; the expert weight gradients then go to the masters, as
     fp32 (the gradients of autocast's casts, computed without a cast pass).
     Returns (y, idx64, weights_x, counts)."""
+    if isinstance(x, torch.Tensor) and x.is_cuda and len(w1) == len(w2) == len(w3) and len(sw1) == len(sw2) == len(sw3):
+        out = _eager_layer(_c(x), _c(gate_w), _c(gate_bias), [*w1, *w2, *w3, *sw1, *sw2, *sw3],
+                           list(master_weights) if master_weights is not None else [], len(w1), len(sw1), int(k),
+                           float(route_scale), training)
+        if out is not None:
+            return out
     E, S, I, I_s = check_layer_args(x, gate_w, gate_bias, w1, w2, w3, sw1, sw2, sw3, k)
     _require_gpu(x, gate_w, gate_bias, *w1)
     weights = [*w1, *w2, *w3, *sw1, *sw2, *sw3]
@@ -374,8 +482,7 @@ class _GroupedSwiGLUFn(torch.autograd.Function):
         lib = L.load()
         ws = _ws(lib.dsmoe_grouped_swiglu_workspace_size(d), dev)
         y = torch.empty(N, D, dtype=x_sorted.dtype, device=dev)
-        p1, k1 = L.ptr_array(list(w1.unbind(0))); p2, k2 = L.ptr_array(list(w2.unbind(0)))
-        p3, k3 = L.ptr_array(list(w3.unbind(0)))
+        p1, k1 = L.stack_array(w1); p2, k2 = L.stack_array(w2); p3, k3 = L.stack_array(w3)
         off = _c(expert_offsets.to(torch.int64))
         rc = lib.dsmoe_grouped_swiglu_fwd(L.ptr(x_sorted), p1, p2, p3, L.ptr(sorted_w), L.ptr(off), d, L.ptr(y),
                                           L.ptr(ws), ws.numel(), L.stream_ptr(dev))
@@ -394,7 +501,7 @@ class _GroupedSwiGLUFn(torch.autograd.Function):
         ws = _ws(lib.dsmoe_grouped_swiglu_bwd_workspace_size(d), dev)
         dx = torch.empty_like(x_sorted)
         dw1, dw2, dw3 = torch.empty_like(w1), torch.empty_like(w2), torch.empty_like(w3)
-        arrs = [L.ptr_array(list(t.unbind(0))) for t in (w1, w2, w3, dw1, dw2, dw3)]
+        arrs = [L.stack_array(t) for t in (w1, w2, w3, dw1, dw2, dw3)]
         rc = lib.dsmoe_grouped_swiglu_bwd(L.ptr(x_sorted), arrs[0][0], arrs[1][0], arrs[2][0], L.ptr(off),
                                           L.ptr(_c(dy)), d, L.ptr(dx), arrs[3][0], arrs[4][0], arrs[5][0], L.ptr(ws),
                                           ws.numel(), L.stream_ptr(dev))
