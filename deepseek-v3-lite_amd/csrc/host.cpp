@@ -11,12 +11,17 @@
 // (inter width, shared inter width, whether anything requires grad, the six host
 // arrays of weight addresses as bytes).
 // addresses(tensors) returns the data pointers of a list of tensors as bytes.
+// empty_like(tensors, float32) returns new tensors of their shapes (contiguous, on
+// their device, in their dtype or float32).
 #include <Python.h>
 
 #include <cstdint>
 #include <cstring>
+#include <utility>
+#include <vector>
 
 #include <ATen/core/Tensor.h>
+#include <ATen/ops/empty.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -131,7 +136,39 @@ PyObject* addresses(PyObject*, PyObject* list) {
   END_HANDLE_TH_ERRORS
 }
 
-PyMethodDef methods[] = {{"scan", scan, METH_VARARGS, nullptr}, {"addresses", addresses, METH_O, nullptr}, {}};
+PyObject* empty_like(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  PyObject* list;
+  int f32;
+  if (!PyArg_ParseTuple(args, "O!p", &PyList_Type, &list, &f32)) return nullptr;
+  const Py_ssize_t n = PyList_GET_SIZE(list);
+  for (Py_ssize_t i = 0; i < n; ++i)
+    if (!THPVariable_Check(PyList_GET_ITEM(list, i))) {
+      PyErr_SetString(PyExc_TypeError, "empty_like: a list of tensors");
+      return nullptr;
+    }
+  std::vector<at::Tensor> made;
+  made.reserve(n);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    const at::Tensor& t = THPVariable_Unpack(PyList_GET_ITEM(list, i));
+    made.push_back(at::empty(t.sizes(), t.options().dtype(f32 ? at::kFloat : t.scalar_type()).requires_grad(false)));
+  }
+  PyObject* out = PyList_New(n);
+  if (!out) return nullptr;
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* o = THPVariable_Wrap(std::move(made[i]));
+    if (!o) {
+      Py_DECREF(out);
+      return nullptr;
+    }
+    PyList_SET_ITEM(out, i, o);
+  }
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {{"scan", scan, METH_VARARGS, nullptr}, {"addresses", addresses, METH_O, nullptr},
+                         {"empty_like", empty_like, METH_VARARGS, nullptr}, {}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

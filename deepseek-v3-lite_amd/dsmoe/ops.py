@@ -311,26 +311,24 @@ def _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, route_scale, train
 
 
 class _LayerFn(torch.autograd.Function):
-    """The eager layer under autograd: as dsmoe::moe_fwd / dsmoe::moe_bwd."""
+    """The eager layer under autograd: as dsmoe::moe_fwd / dsmoe::moe_bwd.  leaves
+    are the weights, or with masters the masters (weights: their copies)."""
 
     @staticmethod
-    def forward(ctx, meta, arrays, x, gate_w, gate_bias, *tensors):
-        E, S, k, I, I_s, rs, training = meta
-        n = 3 * (E + S)
-        y, idx64, wx, counts, ws = _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, rs, training)
-        ctx.meta = (*meta, len(tensors) - n)
-        ctx.save_for_backward(x, gate_w, ws, *tensors[:n])
+    def forward(ctx, meta, arrays, weights, masters, x, gate_w, gate_bias, *leaves):
+        y, idx64, wx, counts, ws = _eager_fwd(x, gate_w, gate_bias, arrays, *meta)
+        ctx.meta = (*meta, masters)
+        ctx.save_for_backward(x, gate_w, ws, *(weights if masters else leaves))
         ctx.set_materialize_grads(False)   # only y carries a gradient
         return y, idx64, wx, counts
 
     @staticmethod
     @once_differentiable
     def backward(ctx, dy, _didx, _dwx, _dcounts):
-        E, S, k, I, I_s, rs, training, n_masters = ctx.meta
+        E, S, k, I, I_s, rs, training, masters = ctx.meta
         x, gate_w, ws, *weights = ctx.saved_tensors
-        n = len(weights)
         if dy is None:
-            return (None,) * (5 + n + n_masters)
+            return (None,) * (7 + len(weights))
         if not training:
             raise RuntimeError("dsmoe: forward ran without saving activations for backward")
         dy = _c(dy)
@@ -339,7 +337,7 @@ class _LayerFn(torch.autograd.Function):
         # was given; those go through the operator, as do the observers' calls
         found = host.scan(weights, [], x, gate_w, None, E, S, k) if _plain_eager() else None
         if found is None or found[:2] != (I, I_s) or ws.device != x.device or not ws.is_contiguous():
-            g = moe_bwd_op(x, gate_w, weights, dy, ws, E, S, k, I, I_s, rs, n_masters > 0)
+            g = moe_bwd_op(x, gate_w, weights, dy, ws, E, S, k, I, I_s, rs, masters)
             dx, dgw, dws = g[0], g[1], g[2:]
         else:
             dev = x.device
@@ -348,18 +346,13 @@ class _LayerFn(torch.autograd.Function):
             bws = _ws(L.load().dsmoe_moe_bwd_workspace_size(d), dev)
             dx = torch.empty_like(x)
             dgw = torch.empty(E, D, dtype=torch.float32, device=dev)
-            if n_masters:
-                dws = [torch.empty_like(w, dtype=torch.float32) for w in weights]
-            else:
-                dws = [torch.empty_like(w) for w in weights]
+            dws = host.empty_like(weights, masters)
             rc = bwd(x.data_ptr(), gate_w.data_ptr(), *found[3], d, dy.data_ptr(), ws.data_ptr(), dx.data_ptr(),
                      dgw.data_ptr(), *[host.addresses(a) for a in _layer_weights(dws, E, S)],
-                     L.DSMOE_F32 if n_masters else L.dtype_code(x.dtype), bws.data_ptr(), bws.numel(),
+                     L.DSMOE_F32 if masters else L.dtype_code(x.dtype), bws.data_ptr(), bws.numel(),
                      L.stream_ptr(dev))
             L.check(rc, "dsmoe_moe_bwd_ex")
-        if n_masters:
-            return (None, None, dx, dgw, None, *([None] * n), *dws)
-        return (None, None, dx, dgw, None, *dws)
+        return (None, None, None, None, dx, dgw, None, *dws)
 
 
 def _eager_layer(x, gate_w, gate_bias, weights, masters, E, S, k, route_scale, training):
@@ -376,7 +369,8 @@ def _eager_layer(x, gate_w, gate_bias, weights, masters, E, S, k, route_scale, t
         training = grad
     if not grad:
         return _eager_fwd(x, gate_w, gate_bias, arrays, E, S, k, I, I_s, route_scale, training)[:4]
-    return _LayerFn.apply((E, S, k, I, I_s, route_scale, bool(training)), arrays, x, gate_w, gate_bias, *weights, *masters)
+    return _LayerFn.apply((E, S, k, I, I_s, route_scale, bool(training)), arrays, weights if masters else None,
+                          bool(masters), x, gate_w, gate_bias, *(masters or weights))
 
 
 def check_layer_args(x: torch.Tensor, gate_w: torch.Tensor, gate_bias: torch.Tensor, w1: Sequence[torch.Tensor],
