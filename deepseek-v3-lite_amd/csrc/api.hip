@@ -351,6 +351,30 @@ int dsmoe_permute_noalloc(const int32_t* idx, const dsmoe_dims* dims, int32_t* o
                        ws, DSMOE_PERMUTE_NOALLOC_BYTES, stream);
 }
 
+// Few-row GEMM path.  Inference calls of at most SK_MAX_T tokens take it for
+// both GEMMs.  Above that the 256-row tiles of the persistent kernel stay mostly
+// padding while the rows of an expert are few: a launch is a stream of weights
+// there, and what counts is how evenly its tiles fill the 256 CUs.
+// few_rows(rows, groups, n): whether the few-row kernel is the faster one for
+// `rows` routed rows over `groups` experts, n output columns (SwiGLU: 2 I).
+// Measured (us, persistent kernel against few-row kernel):
+//   E 16, D 1024, I 512, k 4 (64 tiles of 256 columns, rows per expert 25 / 50 / 83):
+//     gate/up 22 / 27 / 29 against 19 / 23 / 30, down 22 / 28 / 29 against 18 / 19 / 20;
+//   E 20, D 768, I 384, k 4 (60 tiles; 20 / 40 / 67 / 102 rows):
+//     gate/up 18 / 24 / 25 / 25 against 16 / 18 / 20 / 26, down 15 / 19 / 20 / 20 against 12 / 13 / 14 / 21;
+//   E 64, D 2048, I 1408, k 6, down (512 tiles and 16 long ones, a third round of
+//     CUs nearly empty; 9 / 19 / 31 / 48 rows): 122 / 137 / 142 / 143 against 91 / 105 / 121 / 141;
+//   the same, gate/up (704 tiles: 2.75 rounds, 5 TB/s): 143 / 146 / 150 / 154 against 164 / 194 / 225 / 257.
+constexpr int SK_MAX_T = SK_BM;
+
+static bool few_rows(int64_t rows, int groups, int n) {
+  const int64_t tiles = cdiv(n, 256) * groups;
+  if (tiles < 256) return rows <= 64 * (int64_t)groups;
+  // a last round of CUs less than a quarter full: the long tail costs more than re-read activations
+  const int64_t last = tiles % 256;
+  return last < 64 && tiles < 1024 && rows <= 40 * (int64_t)groups;
+}
+
 static size_t grouped_ws(const dsmoe_dims& d, void* base, const void*** ptrs, int32_t** off32, MTile** sched,
                          int32_t** cnt, void** h) {
   Carver c(base);
@@ -405,8 +429,12 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g.sched_count = g2.sched_count = cnt;
   g.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(d.T, d.E, bm);
   g.bm = g2.bm = bm;
-  rc = launch_grouped_gemm(g, EPI_SWIGLU, d.dtype, nullptr, al, st);
+  if (mfr && few_rows(d.T, d.E, 2 * d.I) && gemm_sk_ok(g))
+    rc = launch_gemm_sk(g, EPI_SWIGLU, nullptr, st);
+  else
+    rc = launch_grouped_gemm(g, EPI_SWIGLU, d.dtype, nullptr, al, st);
   if (rc) return rc;
+  if (mfr && few_rows(d.T, d.E, d.D) && gemm_sk_ok(g2)) return launch_gemm_sk(g2, EPI_STORE, sorted_w, st);
   return launch_grouped_gemm(g2, EPI_STORE, d.dtype, sorted_w, al, st);
 }
 
@@ -422,9 +450,6 @@ size_t dsmoe_moe_fwd_workspace_size(const dsmoe_dims* dims, int training) {
   if (validate(dims, true)) return 0;
   return fwd_layout(*dims, training, nullptr).total;
 }
-
-// Few-row (decode) GEMM path: tokens per inference call up to which it is taken.
-constexpr int SK_MAX_T = SK_BM;
 
 // Routed problem gr on the few-row kernel, with the dense shared problem gd
 // in the same launch when that kernel takes it too (else on the general path).
@@ -487,16 +512,21 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   g2.N = d.D; g2.K = d.I; g2.C = L.o_sorted; g2.ldc = d.D;
   const bool mfr = gemm_mfma_eligible(g1, d.dtype, mf) && gemm_mfma_eligible(g2, d.dtype, mf);
   const bool al = d.dtype == DSMOE_F32 ? mf : mfr;
-  // Decode shapes (at most SK_MAX_T tokens, inference): every routed and
-  // shared row tile fits the few-row kernel, which streams the weights once.
-  bool sk = false;
-  if (!training && d.dtype == DSMOE_BF16 && d.T <= SK_MAX_T && mf) {
+  // few rows per expert: the few-row kernel for either GEMM (never where the
+  // gate/up GEMM saves pre-activations)
+  bool sk1 = false, sk2 = false;
+  if (d.dtype == DSMOE_BF16 && mf && (mfr || (!training && d.T <= SK_MAX_T))) {
     GemmDesc t1 = g1, t2 = g2;
     t1.bm = t2.bm = SK_BM;
-    t1.Gs = t1.Us = nullptr;
-    sk = gemm_sk_ok(t1) && gemm_sk_ok(t2);
+    const bool ok1 = !training && gemm_sk_ok(t1), ok2 = gemm_sk_ok(t2);
+    if (d.T <= SK_MAX_T && ok1 && ok2) {
+      sk1 = sk2 = true;
+    } else if (mfr) {
+      sk1 = ok1 && few_rows(N, d.E, 2 * d.I);
+      sk2 = ok2 && few_rows(N, d.E, d.D);
+    }
   }
-  const int bm = sk ? SK_BM : gemm_tile_m(mfr);
+  const int bm = sk1 && sk2 ? SK_BM : gemm_tile_m(mfr);
   // (a) gate; the MFMA gate's routing launch also ranks the slots for the
   // permute (and finishes it for a call of one rank block)
   const PermuteOut po = permute_out(L.ps, bm, L.offsets, L.sorted_slot, L.sorted_token, L.slot_pos, counts,
@@ -541,9 +571,8 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
     s2.N = d.D; s2.K = d.S * d.I_s; s2.C = L.shared_out; s2.ldc = d.D;
     s2.bm = gemm_tile_m(gemm_mfma_eligible(s2, d.dtype, mf));
   }
-  if (sk) g1.Gs = g1.Us = s1.Gs = s1.Us = nullptr;  // inference: no pre-activation saves
   tm.begin(ST_GEMM1);
-  rc = sk ? launch_sk_pair(g1, s1, d.S > 0, EPI_SWIGLU, d.dtype, mf, st)
+  rc = sk1 ? launch_sk_pair(g1, s1, d.S > 0, EPI_SWIGLU, d.dtype, mf, st)
           : d.S ? launch_grouped_gemm_pair(g1, s1, EPI_SWIGLU, d.dtype, nullptr, al, mf, st)
                 : launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, al, st);
   tm.end();
@@ -552,7 +581,7 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   // o_sorted is sorted position r); the combine and the backward read slot s
   // at row slot_pos[s]
   tm.begin(ST_GEMM2);
-  rc = sk ? launch_sk_pair(g2, s2, d.S > 0, EPI_STORE, d.dtype, mf, st)
+  rc = sk2 ? launch_sk_pair(g2, s2, d.S > 0, EPI_STORE, d.dtype, mf, st)
           : d.S ? launch_grouped_gemm_pair(g2, s2, EPI_STORE, d.dtype, nullptr, al, mf, st)
                 : launch_grouped_gemm(g2, EPI_STORE, d.dtype, nullptr, al, st);
   tm.end();

@@ -229,8 +229,8 @@ int launch_gemm_f32(const GemmDesc& gr, const GemmDesc* gd, int epi, const float
 int launch_xgemm_f32(const XGemm& g, int epi, bool tables_aligned, hipStream_t st);
 // K parts (1, 2, 4 or 8) of a dense fp32 weight gradient of groups x M x N outputs over k_len rows.
 int xgemm_f32_ksplit(int64_t M, int64_t N, int groups, int64_t k_len);
-// Few-row grouped GEMM (decode): row tiles of SK_BM rows, weights streamed
-// once.  The routed schedule must be built with bm = SK_BM; no G/U saves.
+// Few-row grouped GEMM: row tiles of SK_BM rows, weights streamed once for each.
+// The routed schedule's height is a multiple of SK_BM; no G/U saves.
 constexpr int SK_BM = 64;
 bool gemm_sk_ok(const GemmDesc& g);
 int launch_gemm_sk(const GemmDesc& g, int epi, const float* row_scale, hipStream_t st);

@@ -18,7 +18,7 @@
 // 16-byte chunks.
 //
 // Tile enumeration (gemm_tile.h) and GemmDesc contract as in gemm.hip, with row tiles of
-// SK_BM rows (the routed schedule must be built with bm = SK_BM).
+// SK_BM rows (the routed schedule's height is a multiple of SK_BM).
 #include "gemm_tile.h"
 #include "mfma.h"
 
@@ -197,14 +197,14 @@ __global__ __launch_bounds__(256) void gemm_sk_kernel(const GemmDesc g0, const G
 // ---------------------------------------------------------------- host side
 bool gemm_sk_ok(const GemmDesc& g) {
   const auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  const bool rows_ok = g.sched ? g.bm == SK_BM : g.dense_rows >= 0;
+  const bool rows_ok = g.sched ? g.bm % SK_BM == 0 : g.dense_rows >= 0;
   return rows_ok && g.nseg >= 1 && g.nseg <= 2 && g.K > 0 && g.K % (4 * SK_KSTEP) == 0 && g.kseg % SK_KSTEP == 0 &&
          g.N > 0 && g.N % 8 == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 8 == 0 && g.c_group_col % 8 == 0 &&
          a16(g.A) && a16(g.C) && g.Gs == nullptr && g.Us == nullptr;
 }
 
 static int64_t sk_mtiles(const GemmDesc& g) {
-  return g.sched ? g.m_tiles_bound : cdiv(g.dense_rows, SK_BM) * g.groups;
+  return g.sched ? (int64_t)g.m_tiles_bound * (g.bm / SK_BM) : cdiv(g.dense_rows, SK_BM) * g.groups;
 }
 
 template <int EPI>

@@ -7,14 +7,17 @@ namespace dsmoe {
 
 // Maps blockIdx.x to (group, first row, valid rows, N tile).  Tiles are
 // enumerated M-major, N fastest; block b runs on XCD b % 8 and XCD x takes the
-// x-th contiguous eighth of the tile list.  Returns false for surplus blocks.
+// x-th contiguous eighth of the tile list.  A routed schedule of height bm (a
+// multiple of BM) is cut into bm / BM tiles an entry.  Returns false for surplus
+// blocks and for the parts of an entry past its rows.
 template <int BM>
 __device__ __forceinline__ bool tile_for_block(const GemmDesc& g, int n_tiles, int& grp, int& row0, int& rows,
                                                int& n_tile) {
   int64_t m_total;
   int tpg = 0;
+  const int sub = g.sched ? g.bm / BM : 1;
   if (g.sched) {
-    m_total = *g.sched_count;
+    m_total = (int64_t)*g.sched_count * sub;
   } else {
     tpg = (int)cdiv(g.dense_rows, BM);
     m_total = (int64_t)tpg * g.groups;
@@ -28,10 +31,12 @@ __device__ __forceinline__ bool tile_for_block(const GemmDesc& g, int n_tiles, i
   const int64_t m_tile = lin / n_tiles;
   n_tile = (int)(lin - m_tile * n_tiles);
   if (g.sched) {
-    const MTile t = g.sched[m_tile];
+    const MTile t = g.sched[m_tile / sub];
+    const int s = (int)(m_tile % sub) * BM;
     grp = t.group;
-    row0 = t.row0;
-    rows = t.rows;
+    row0 = t.row0 + s;
+    rows = min(BM, t.rows - s);
+    return rows > 0;
   } else {
     grp = (int)(m_tile / tpg);
     const int mt = (int)(m_tile - (int64_t)grp * tpg);
@@ -55,8 +60,9 @@ __device__ __forceinline__ bool tile_for_block_pair(const GemmDesc& gr, const Ge
   const int64_t td = (int64_t)tpg_d * gd.groups * ntd;
   int tpg_r = 0;
   int64_t mr;
+  const int sub = gr.sched ? gr.bm / BM : 1;
   if (gr.sched) {
-    mr = *gr.sched_count;
+    mr = (int64_t)*gr.sched_count * sub;
   } else {
     tpg_r = (int)cdiv(gr.dense_rows, BM);
     mr = (int64_t)tpg_r * gr.groups;
@@ -83,10 +89,12 @@ __device__ __forceinline__ bool tile_for_block_pair(const GemmDesc& gr, const Ge
   const int64_t m_tile = lin / ntr;
   n_tile = (int)(lin - m_tile * ntr);
   if (gr.sched) {
-    const MTile t = gr.sched[m_tile];
+    const MTile t = gr.sched[m_tile / sub];
+    const int s = (int)(m_tile % sub) * BM;
     grp = t.group;
-    row0 = t.row0;
-    rows = t.rows;
+    row0 = t.row0 + s;
+    rows = min(BM, t.rows - s);
+    return rows > 0;
   } else {
     grp = (int)(m_tile / tpg_r);
     row0 = (int)(m_tile - (int64_t)grp * tpg_r) * BM;

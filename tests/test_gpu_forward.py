@@ -462,3 +462,28 @@ def test_update_bias_with_fractional_counts():
     assert torch.equal(gate.bias.cpu(), R.update_bias_ref(b0, counts, 0.01))
     truncated = R.update_bias_ref(b0, counts.to(torch.int32), 0.01)
     assert not torch.equal(gate.bias.cpu(), truncated)             # integer truncation would differ
+
+
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("case,skew", [
+    (CS.Case("few_unfilled", 65, 256, 16, 128, 2, 1, 128, torch.bfloat16, "normal"), False),   # both GEMMs few-row
+    (CS.Case("few_unfilled", 190, 256, 4, 256, 1, 1, 128, torch.bfloat16), True),   # one expert with every row: 64-row parts
+    (CS.Case("few_unfilled", 256, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False),  # at the line: 64 rows each
+    (CS.Case("few_down", 70, 2048, 64, 256, 4, 2, 256, torch.bfloat16, "normal"), False),   # the down projection alone
+], ids=lambda c: str(c) if isinstance(c, bool) else f"{c.name}_T{c.T}")
+def test_few_rows_per_expert(case, skew, training):
+    """More than 64 tokens with few rows per expert: the few-row GEMM on schedules of its own height and of 256 rows,
+    beside the persistent one."""
+    x, p, _ = CS.make_inputs(case)
+    if skew:
+        p = R.MoEParams(p.gate_w, torch.tensor([0.0, 5.0, 0.0, 0.0]), p.w1, p.w2, p.w3, p.sw1, p.sw2, p.sw3)
+    q = CS.params_to(p, DEV)
+    from dsmoe import moe_layer
+    with torch.no_grad():
+        y, idx, _, counts = moe_layer(x.to(DEV), q.gate_w, q.gate_bias, q.w1, q.w2, q.w3, q.sw1, q.sw2, q.sw3, k=case.k,
+                                      training=training)
+    torch.cuda.synchronize()
+    if skew:
+        assert counts.tolist() == [0, case.T, 0, 0]
+    ref = R.moe_forward_ref(x, p, case.k, indices=idx.cpu())
+    torch.testing.assert_close(y.cpu().float(), ref.float(), rtol=2e-2, atol=2e-2)
