@@ -48,9 +48,13 @@ struct MlaArgs {
   const bf16_t* q_pe;     // (B, H, S_q, Dr)
   const bf16_t* ctx_kv;   // (B, S_kv, R)
   const bf16_t* ctx_pe;   // (B, S_kv, Dr)
-  const bf16_t* w_k;      // (H, Dn, R)
-  const bf16_t* w_v;      // (H, Dv, R)
+  const bf16_t* w_k;      // head h's (Dn, R) rows at h wk_hs
+  const bf16_t* w_v;      // head h's (Dv, R) rows at h wv_hs
+  int64_t wk_hs, wv_hs;
   bf16_t* out;            // (B, S_q, H, Dv)
+  int nsp;                // key ranges of the forward, each its own workgroup (mla_splits)
+  float* po;              // nsp > 1: (B, H, nsp, S_q, DVp) unnormalised outputs
+  float2* pml;            // nsp > 1: (B, H, nsp, S_q) {max score, sum of p}
   float* lse;             // (B, H, S_q): c m + log2(sum of p), the base-2 log-sum-exp of the scaled scores, or null
   // backward
   const bf16_t* dout;     // (B, S_q, H, Dv)
@@ -179,8 +183,8 @@ __global__ __launch_bounds__(256) void mla_kv_kernel(const MlaArgs a) {
         const int i = min(tid + 256 * u, tot - 1);
         const int r = i / cpr, c = i - r * cpr;
         const int nc = min(n0 + r, ncols - 1);
-        const bf16_t* wrow = nc < a.Dn ? a.w_k + ((int64_t)h * a.Dn + nc) * a.R
-                                       : a.w_v + ((int64_t)h * a.Dv + (nc - a.Dn)) * a.R;
+        const bf16_t* wrow = nc < a.Dn ? a.w_k + (int64_t)h * a.wk_hs + (int64_t)nc * a.R
+                                       : a.w_v + (int64_t)h * a.wv_hs + (int64_t)(nc - a.Dn) * a.R;
         wv[u] = *reinterpret_cast<const mla_u32x4*>(wrow + min(c * 8, a.R - 8));
       }
 #pragma unroll
@@ -206,8 +210,8 @@ __global__ __launch_bounds__(256) void mla_kv_kernel(const MlaArgs a) {
           fw[ks] = *reinterpret_cast<const bf16x8_t*>(sw + (32 * t + l32) * rs + (16 * ks + 8 * hi) * 2);
       } else {
         const int nc = min(n, ncols - 1);
-        const bf16_t* wrow = nc < a.Dn ? a.w_k + ((int64_t)h * a.Dn + nc) * a.R
-                                       : a.w_v + ((int64_t)h * a.Dv + (nc - a.Dn)) * a.R;
+        const bf16_t* wrow = nc < a.Dn ? a.w_k + (int64_t)h * a.wk_hs + (int64_t)nc * a.R
+                                       : a.w_v + (int64_t)h * a.wv_hs + (int64_t)(nc - a.Dn) * a.R;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
           if (ks < nks) fw[ks] = frag(wrow, n < ncols, 16 * ks + 8 * hi);
@@ -333,7 +337,8 @@ struct MlaCfg {
 };
 
 // Work items (batch, head, query block) as mla_item orders them, a pair's
-// query blocks last-first (causal: the longest first).
+// query blocks last-first (causal: the longest first).  With nsp > 1 an item is
+// one of nsp equal ranges of the block's keys; mla_merge_kernel adds them.
 template <int NSTEP, int NV>
 __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
   using C = MlaCfg<NSTEP, NV>;
@@ -342,9 +347,10 @@ __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
   const int hi = lane >> 5, ql = lane & 31;
   const int nq = (a.S_q + MLA_QB - 1) / MLA_QB;
   int hb, rank;
-  if (!mla_item((int)blockIdx.x, a.B * a.H, nq, hb, rank)) return;
+  if (!mla_item((int)blockIdx.x, a.B * a.H, nq * a.nsp, hb, rank)) return;
   const int h = hb % a.H, b = hb / a.H;
-  const int q0 = (nq - 1 - rank) * MLA_QB;
+  const int split = rank % a.nsp;
+  const int q0 = (nq - 1 - rank / a.nsp) * MLA_QB;
   const int qi = q0 + 32 * wave + ql;          // this lane's query
   const int64_t bh = (int64_t)b * a.H + h;
 
@@ -399,7 +405,8 @@ __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
   // keys this workgroup needs
   int kend = a.S_kv;
   if (a.causal) kend = min(kend, min(q0 + MLA_QB, a.S_q) - 1 + a.q_start + 1);
-  const int nkb = (kend + MLA_KB - 1) / MLA_KB;
+  const int nkb_all = (kend + MLA_KB - 1) / MLA_KB;
+  const int kb0 = (int)((int64_t)nkb_all * split / a.nsp), nkb = (int)((int64_t)nkb_all * (split + 1) / a.nsp);
   const char* kg = reinterpret_cast<const char*>(a.kbuf + bh * a.S_kvp * C::DQKp);
   const char* vg = reinterpret_cast<const char*>(a.vbuf + bh * a.S_kvp * C::DVp);
   const int wv = __builtin_amdgcn_readfirstlane(wave);
@@ -438,8 +445,8 @@ __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
   float m = -INFINITY, l = 0.0f;
   const int qpos = qi + a.q_start;
 
-  if (nkb > 0) issue(0);
-  for (int kb = 0; kb < nkb; ++kb) {
+  if (kb0 < nkb) issue(kb0);
+  for (int kb = kb0; kb < nkb; ++kb) {
     // block kb has landed for every wave, and every wave is done with block kb - 1
     wait_vm<0>();
     wait_lgkm0();
@@ -537,6 +544,18 @@ __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
   const float lt = mla_pair_sum(l);
   const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
   if (qi >= a.S_q) return;
+  if (a.nsp > 1) {
+    const int64_t pr = (bh * a.nsp + split) * a.S_q + qi;
+    if (hi == 0) a.pml[pr] = make_float2(m, lt);
+    float* pw = a.po + pr * C::DVp;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4*>(pw + 32 * v + 8 * g + 4 * hi) =
+            make_float4(o[v][4 * g], o[v][4 * g + 1], o[v][4 * g + 2], o[v][4 * g + 3]);
+    return;
+  }
   // the backward's probabilities are exp2(c s - lse); a query without a
   // visible key gets +inf (probability 0)
   if (a.lse && hi == 0) a.lse[bh * a.S_q + qi] = lt > 0.0f ? m * a.c + log2f(lt) : INFINITY;
@@ -562,6 +581,53 @@ __global__ __launch_bounds__(256) void mla_fa_kernel(const MlaArgs a) {
           if (dv + e < a.Dv) orow[dv + e] = f2bf(o[v][4 * g + e] * inv);
       }
     }
+}
+
+// The key ranges of a query added by their weights exp2(c (m_i - max m)): DVp / 4
+// lanes per (batch, head, query).
+constexpr int MLA_MAX_SPLITS = 16;
+
+__global__ __launch_bounds__(256) void mla_merge_kernel(const MlaArgs a) {
+  const int lanes = a.DVp / 4;
+  const int64_t row = (int64_t)blockIdx.x * (256 / lanes) + threadIdx.x / lanes;
+  const int dv = 4 * (threadIdx.x % lanes);
+  if (row >= (int64_t)a.B * a.H * a.S_q) return;
+  const int64_t bh = row / a.S_q;
+  const int qi = (int)(row - bh * a.S_q);
+  const int h = (int)(bh % a.H), b = (int)(bh / a.H);
+  const int64_t p0 = bh * a.nsp * a.S_q + qi;
+  float2 ml[MLA_MAX_SPLITS];
+  float4 v[MLA_MAX_SPLITS];
+#pragma unroll
+  for (int i = 0; i < MLA_MAX_SPLITS; ++i) {
+    const int64_t p = p0 + (int64_t)min(i, a.nsp - 1) * a.S_q;
+    ml[i] = a.pml[p];
+    v[i] = *reinterpret_cast<const float4*>(a.po + p * a.DVp + dv);
+  }
+  float m = -INFINITY, l = 0.0f;
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+  for (int i = 0; i < MLA_MAX_SPLITS; ++i) m = fmaxf(m, ml[i].x);
+#pragma unroll
+  for (int i = 0; i < MLA_MAX_SPLITS; ++i) {
+    const float w = i < a.nsp && ml[i].y > 0.0f ? __builtin_amdgcn_exp2f((ml[i].x - m) * a.c) : 0.0f;
+    l = fmaf(w, ml[i].y, l);
+    o.x = fmaf(w, v[i].x, o.x);
+    o.y = fmaf(w, v[i].y, o.y);
+    o.z = fmaf(w, v[i].z, o.z);
+    o.w = fmaf(w, v[i].w, o.w);
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  if (a.lse && dv == 0) a.lse[row] = l > 0.0f ? m * a.c + log2f(l) : INFINITY;
+  bf16_t* orow = a.out + (((int64_t)b * a.S_q + qi) * a.H + h) * a.Dv + dv;
+  const float f[4] = {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
+  if (a.ovec && dv + 3 < a.Dv) {
+    *reinterpret_cast<u32x2_t*>(orow) = u32x2_t{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])};
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (dv + e < a.Dv) orow[e] = f2bf(f[e]);
+  }
 }
 
 // ---------------------------------------------------------------- backward
@@ -1141,6 +1207,23 @@ static int mla_validate(const dsmoe_mla_dims* d) {
   return DSMOE_OK;
 }
 
+// Key ranges of the forward: more than one where its workgroups (128 queries of a
+// (batch, head)) leave half of the CUs idle, so that there are about 512, each with
+// two key blocks or more (256 to 768 measure the same).  At H 12, D_nope 48,
+// D_rope 24, D_v 64, B 1 (us, one range against this, with the K, V launch): 500
+// queries of 1300 keys 37 -> 31 (attention 28.6 -> 15.5, sum 5.6), 128 of 2048 51 -> 28,
+// 40 of 1300 36 -> 22; 192 workgroups (B 2, 1024 of 1024) 36 -> 43 with two ranges.
+static int mla_splits(const MlaArgs& a) {
+  const int64_t items = (int64_t)a.B * a.H * cdiv(a.S_q, MLA_QB);
+  if (items >= 128) return 1;
+  const int64_t n = std::min<int64_t>({MLA_MAX_SPLITS, 512 / items, cdiv(a.S_kv, MLA_KB) / 2});
+  return (int)std::max<int64_t>(1, n);
+}
+
+static size_t mla_kv_bytes(const MlaArgs& a) {
+  return align_up((size_t)a.B * a.H * a.S_kvp * (a.DQKp + a.DVp) * sizeof(bf16_t), 256);
+}
+
 static MlaArgs mla_args(const dsmoe_mla_dims* d) {
   MlaArgs a;
   std::memset(static_cast<void*>(&a), 0, sizeof(a));
@@ -1157,6 +1240,7 @@ static MlaArgs mla_args(const dsmoe_mla_dims* d) {
   a.negq = d->softmax_scale < 0.0f ? 1 : 0;
   a.c = (d->softmax_scale < 0.0f ? -d->softmax_scale : d->softmax_scale) * MLA_LOG2E;
   a.scale = d->softmax_scale;
+  a.nsp = mla_splits(a);
   return a;
 }
 
@@ -1170,8 +1254,12 @@ static int mla_launch_fa(const MlaArgs& a, hipStream_t st) {
         hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (attr != hipSuccess) return fail(DSMOE_ERR_HIP, "mla: cannot raise LDS limit");
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)mla_grid(a.B * a.H, (int)cdiv(a.S_q, MLA_QB))), dim3(256), lds, st, a);
-  return check_launch("mla_fa");
+  hipLaunchKernelGGL(kern, dim3((unsigned)mla_grid(a.B * a.H, (int)cdiv(a.S_q, MLA_QB) * a.nsp)), dim3(256), lds, st, a);
+  const int rc = check_launch("mla_fa");
+  if (rc || a.nsp == 1) return rc;
+  const int64_t rows = (int64_t)a.B * a.H * a.S_q;
+  hipLaunchKernelGGL(mla_merge_kernel, dim3((unsigned)cdiv(rows, 256 / (a.DVp / 4))), dim3(256), 0, st, a);
+  return check_launch("mla_merge");
 }
 
 template <int NSTEP>
@@ -1241,7 +1329,8 @@ static int mla_launch_kv(const MlaArgs& a, hipStream_t st) {
 
 // The forward's operands, vector-load flags and K, V buffers of a call.
 static MlaArgs mla_bind(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
-                        const void* wkv_b_k, const void* wkv_b_v, const dsmoe_mla_dims* dims, void* workspace) {
+                        const void* wkv_b_k, int64_t wk_hs, const void* wkv_b_v, int64_t wv_hs,
+                        const dsmoe_mla_dims* dims, void* workspace) {
   MlaArgs a = mla_args(dims);
   a.q_nope = static_cast<const bf16_t*>(q_nope);
   a.q_pe = static_cast<const bf16_t*>(q_pe);
@@ -1251,10 +1340,17 @@ static MlaArgs mla_bind(const void* q_nope, const void* q_pe, const void* ctx_kv
   a.w_v = static_cast<const bf16_t*>(wkv_b_v);
   auto al = [](const void* p, uintptr_t m) { return (reinterpret_cast<uintptr_t>(p) & (m - 1)) == 0; };
   a.qvec = (a.Dn % 8 == 0 && a.Dr % 8 == 0 && al(q_nope, 16) && al(q_pe, 16)) ? 1 : 0;
-  a.kvvec = (a.R % 8 == 0 && al(ctx_kv, 16) && al(wkv_b_k, 16) && al(wkv_b_v, 16)) ? 1 : 0;
+  a.wk_hs = wk_hs;
+  a.wv_hs = wv_hs;
+  a.kvvec = (a.R % 8 == 0 && wk_hs % 8 == 0 && wv_hs % 8 == 0 && al(ctx_kv, 16) && al(wkv_b_k, 16) &&
+             al(wkv_b_v, 16)) ? 1 : 0;
   a.pevec = (a.Dn % 8 == 0 && a.Dr % 8 == 0 && al(ctx_pe, 16)) ? 1 : 0;
   a.kbuf = static_cast<bf16_t*>(workspace);
   a.vbuf = a.kbuf + (size_t)a.B * a.H * a.S_kvp * a.DQKp;
+  if (a.nsp > 1) {   // after K and V
+    a.po = reinterpret_cast<float*>(static_cast<char*>(workspace) + mla_kv_bytes(a));
+    a.pml = reinterpret_cast<float2*>(a.po + (size_t)a.B * a.H * a.nsp * a.S_q * a.DVp);
+  }
   return a;
 }
 
@@ -1265,21 +1361,26 @@ using namespace dsmoe;
 extern "C" size_t dsmoe_mla_attn_workspace_size(const dsmoe_mla_dims* dims) {
   if (mla_validate(dims) != DSMOE_OK) return 0;
   const MlaArgs a = mla_args(dims);
-  return (size_t)a.B * a.H * a.S_kvp * (a.DQKp + a.DVp) * sizeof(bf16_t) + 256;
+  const size_t parts = a.nsp > 1 ? (size_t)a.B * a.H * a.nsp * a.S_q * (a.DVp + 2) * sizeof(float) : 0;
+  return mla_kv_bytes(a) + parts + 256;
 }
 
 static int mla_fwd(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe, const void* wkv_b_k,
-                   const void* wkv_b_v, const dsmoe_mla_dims* dims, void* out, float* lse, void* workspace,
-                   size_t workspace_bytes, void* stream) {
+                   int64_t wk_hs, const void* wkv_b_v, int64_t wv_hs, const dsmoe_mla_dims* dims, void* out, float* lse,
+                   void* workspace, size_t workspace_bytes, void* stream) {
   int rc = mla_validate(dims);
   if (rc) return rc;
   DSMOE_REQUIRE(q_nope && q_pe && ctx_kv && ctx_pe && wkv_b_k && wkv_b_v && out, DSMOE_ERR_INVALID,
                 "mla: NULL tensor pointer");
   const size_t need = dsmoe_mla_attn_workspace_size(dims);
-  DSMOE_REQUIRE(workspace && workspace_bytes >= need, DSMOE_ERR_WORKSPACE, "mla: workspace too small");
+  // K and V must fit; a workspace sized for a larger call (one that needs no key
+  // ranges) takes this one without ranges
+  DSMOE_REQUIRE(workspace && workspace_bytes >= mla_kv_bytes(mla_args(dims)) + 256, DSMOE_ERR_WORKSPACE,
+                "mla: workspace too small");
   DSMOE_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, DSMOE_ERR_INVALID,
                 "mla: workspace must be 16-byte aligned");
-  MlaArgs a = mla_bind(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, dims, workspace);
+  MlaArgs a = mla_bind(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wk_hs, wkv_b_v, wv_hs, dims, workspace);
+  if (workspace_bytes < need) a.nsp = 1;
   a.out = static_cast<bf16_t*>(out);
   a.lse = lse;
   a.ovec = (a.Dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0) ? 1 : 0;
@@ -1299,15 +1400,27 @@ static int mla_fwd(const void* q_nope, const void* q_pe, const void* ctx_kv, con
 extern "C" int dsmoe_mla_attn_fwd(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
                                   const void* wkv_b_k, const void* wkv_b_v, const dsmoe_mla_dims* dims, void* out,
                                   void* workspace, size_t workspace_bytes, void* stream) {
-  return mla_fwd(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, dims, out, nullptr, workspace, workspace_bytes,
-                 stream);
+  const int64_t r = dims ? dims->R : 0;
+  return mla_fwd(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, r * (dims ? dims->D_nope : 0), wkv_b_v,
+                 r * (dims ? dims->D_v : 0), dims, out, nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dsmoe_mla_attn_fwd_lse(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
                                       const void* wkv_b_k, const void* wkv_b_v, const dsmoe_mla_dims* dims, void* out,
                                       float* lse, void* workspace, size_t workspace_bytes, void* stream) {
   DSMOE_REQUIRE(lse, DSMOE_ERR_INVALID, "mla: NULL lse pointer");
-  return mla_fwd(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, dims, out, lse, workspace, workspace_bytes, stream);
+  const int64_t r = dims ? dims->R : 0;
+  return mla_fwd(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, r * (dims ? dims->D_nope : 0), wkv_b_v,
+                 r * (dims ? dims->D_v : 0), dims, out, lse, workspace, workspace_bytes, stream);
+}
+
+extern "C" int dsmoe_mla_attn_fwd_heads(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
+                                        const void* wkv_b_k, int64_t wk_head_stride, const void* wkv_b_v,
+                                        int64_t wv_head_stride, const dsmoe_mla_dims* dims, void* out, float* lse,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  DSMOE_REQUIRE(wk_head_stride >= 0 && wv_head_stride >= 0, DSMOE_ERR_INVALID, "mla: negative weight stride");
+  return mla_fwd(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wk_head_stride, wkv_b_v, wv_head_stride, dims, out, lse,
+                 workspace, workspace_bytes, stream);
 }
 
 // K and V alone: the forward's first launch, for a backward whose caller did
@@ -1317,12 +1430,13 @@ extern "C" int dsmoe_mla_attn_kv(const void* ctx_kv, const void* ctx_pe, const v
   const int rc = mla_validate(dims);
   if (rc) return rc;
   DSMOE_REQUIRE(ctx_kv && ctx_pe && wkv_b_k && wkv_b_v, DSMOE_ERR_INVALID, "mla: NULL tensor pointer");
-  DSMOE_REQUIRE(kv_ws && kv_bytes >= dsmoe_mla_attn_workspace_size(dims), DSMOE_ERR_WORKSPACE,
+  DSMOE_REQUIRE(kv_ws && kv_bytes >= mla_kv_bytes(mla_args(dims)) + 256, DSMOE_ERR_WORKSPACE,
                 "mla: workspace too small");
   DSMOE_REQUIRE((reinterpret_cast<uintptr_t>(kv_ws) & 15) == 0, DSMOE_ERR_INVALID,
                 "mla: workspace must be 16-byte aligned");
   // (no queries: the query-load flag, which K, V do not use, sees ctx_kv)
-  const MlaArgs a = mla_bind(ctx_kv, ctx_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, dims, kv_ws);
+  const MlaArgs a = mla_bind(ctx_kv, ctx_pe, ctx_kv, ctx_pe, wkv_b_k, (int64_t)dims->D_nope * dims->R, wkv_b_v,
+                             (int64_t)dims->D_v * dims->R, dims, kv_ws);
   return mla_launch_kv(a, static_cast<hipStream_t>(stream));
 }
 
@@ -1351,7 +1465,7 @@ extern "C" int dsmoe_mla_attn_bwd(const void* q_nope, const void* q_pe, const ds
   if (rc) return rc;
   DSMOE_REQUIRE(q_nope && q_pe && out && dout && lse, DSMOE_ERR_INVALID, "mla: NULL tensor pointer");
   DSMOE_REQUIRE(dq_nope && dq_pe && dkv && dk_pe, DSMOE_ERR_INVALID, "mla: NULL gradient pointer");
-  DSMOE_REQUIRE(kv_ws && kv_bytes >= dsmoe_mla_attn_workspace_size(dims), DSMOE_ERR_WORKSPACE,
+  DSMOE_REQUIRE(kv_ws && kv_bytes >= mla_kv_bytes(mla_args(dims)) + 256, DSMOE_ERR_WORKSPACE,
                 "mla: K, V workspace too small");
   const size_t need = dsmoe_mla_attn_bwd_workspace_size(dims);
   DSMOE_REQUIRE(workspace && workspace_bytes >= need, DSMOE_ERR_WORKSPACE, "mla: workspace too small");

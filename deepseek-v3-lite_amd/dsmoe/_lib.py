@@ -77,6 +77,7 @@ _SIGNATURES = {
     "dsmoe_mla_attn_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),
     "dsmoe_mla_attn_fwd": ([P, P, P, P, P, P, ctypes.POINTER(MlaDims), P, P, SZ, P], I32),
     "dsmoe_mla_attn_fwd_lse": ([P, P, P, P, P, P, ctypes.POINTER(MlaDims), P, P, P, SZ, P], I32),
+    "dsmoe_mla_attn_fwd_heads": ([P, P, P, P, P, I64, P, I64, ctypes.POINTER(MlaDims), P, P, P, SZ, P], I32),
     "dsmoe_mla_attn_few_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),
     "dsmoe_mla_attn_few": ([P, P, P, P, P, I64, P, I64, ctypes.POINTER(MlaDims), P, P, P, SZ, P], I32),
     "dsmoe_mla_attn_bwd_workspace_size": ([ctypes.POINTER(MlaDims)], SZ),

@@ -99,9 +99,8 @@ def _prepare(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v):
         raise ValueError(f"mla_attention: H * S_kv = {H * S_kv} (H * S_q = {H * S_q}) reaches 2^22, the limit of "
                          "one batch row of the kernels' 32-bit row offsets")
     bc = min(B, (_ROWS_PER_CALL - 1) // per_batch)
-    if _few(S_q, R, D_nope, D_v) and _head_rows(wkv_b_k) and _head_rows(wkv_b_v):
-        return (*(t.contiguous() for t in ts[:4]), wkv_b_k, wkv_b_v), bc
-    return tuple(t.contiguous() for t in ts), bc
+    # weights whose heads are whole rows, at any distance, are read in place
+    return (*(t.contiguous() for t in ts[:4]), *(w if _head_rows(w) else w.contiguous() for w in ts[4:])), bc
 
 
 def _few(S_q: int, R: int, D_nope: int, D_v: int) -> bool:
@@ -133,11 +132,14 @@ def _forward_few(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: in
     out = torch.empty(B, S_q, H, wkv_b_v.size(1), dtype=torch.bfloat16, device=dev)
     lse = torch.empty(B, H, S_q, dtype=torch.float32, device=dev)
     for b0 in range(0, B, bc):
-        b1 = min(B, b0 + bc)
         c = (q_nope, q_pe, ctx_kv, ctx_pe, out, lse)
         if bc < B:
+            b1 = min(B, b0 + bc)
             c = tuple(t[b0:b1] for t in c)
             d.B = b1 - b0
+            nbytes = int(lib.dsmoe_mla_attn_few_workspace_size(d))
+            if nbytes > ws.numel():   # a shorter last chunk may take more key ranges
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         L.check(lib.dsmoe_mla_attn_few(L.ptr(c[0]), L.ptr(c[1]), L.ptr(c[2]), L.ptr(c[3]), L.ptr(wkv_b_k),
                                        wkv_b_k.stride(0), L.ptr(wkv_b_v), wkv_b_v.stride(0), d, L.ptr(c[4]),
                                        L.ptr(c[5]), L.ptr(ws), nbytes, L.stream_ptr(dev)), "dsmoe_mla_attn_few")
@@ -155,7 +157,7 @@ def _forward(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int, w
     D_v = wkv_b_v.size(1)
     dev = q_nope.device
     lib = L.load()
-    d = _dims(q_nope[:bc], q_pe[:bc], ctx_kv[:bc], wkv_b_v, softmax_scale, is_causal, q_start)
+    d = _dims(q_nope[:bc], q_pe, ctx_kv, wkv_b_v, softmax_scale, is_causal, q_start)
     nbytes = int(lib.dsmoe_mla_attn_workspace_size(d))
     if nbytes == 0:
         L.check(lib.dsmoe_mla_attn_fwd(None, None, None, None, None, None, d, None, None, 0, None),
@@ -164,15 +166,18 @@ def _forward(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int, w
     out = torch.empty(B, S_q, H, D_v, dtype=torch.bfloat16, device=dev)
     lse = torch.empty(B, H, S_q, dtype=torch.float32, device=dev) if want_lse else None
     for b0 in range(0, B, bc):
-        b1 = min(B, b0 + bc)
-        d = _dims(q_nope[b0:b1], q_pe[b0:b1], ctx_kv[b0:b1], wkv_b_v, softmax_scale, is_causal, q_start)
-        ins = (L.ptr(q_nope[b0:b1]), L.ptr(q_pe[b0:b1]), L.ptr(ctx_kv[b0:b1]), L.ptr(ctx_pe[b0:b1]),
-               L.ptr(wkv_b_k), L.ptr(wkv_b_v), d, L.ptr(out[b0:b1]))
-        if want_lse:
-            L.check(lib.dsmoe_mla_attn_fwd_lse(*ins, L.ptr(lse[b0:b1]), L.ptr(ws), nbytes, L.stream_ptr(dev)),
-                    "dsmoe_mla_attn_fwd_lse")
-        else:
-            L.check(lib.dsmoe_mla_attn_fwd(*ins, L.ptr(ws), nbytes, L.stream_ptr(dev)), "dsmoe_mla_attn_fwd")
+        c = (q_nope, q_pe, ctx_kv, ctx_pe, out, lse)
+        if bc < B:
+            b1 = min(B, b0 + bc)
+            c = tuple(t[b0:b1] if t is not None else None for t in c)
+            d.B = b1 - b0
+            nbytes = int(lib.dsmoe_mla_attn_workspace_size(d))
+            if nbytes > ws.numel():   # a shorter last chunk may take more key ranges
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        L.check(lib.dsmoe_mla_attn_fwd_heads(L.ptr(c[0]), L.ptr(c[1]), L.ptr(c[2]), L.ptr(c[3]), L.ptr(wkv_b_k),
+                                             wkv_b_k.stride(0), L.ptr(wkv_b_v), wkv_b_v.stride(0), d, L.ptr(c[4]),
+                                             L.ptr(c[5]), L.ptr(ws), nbytes, L.stream_ptr(dev)),
+                "dsmoe_mla_attn_fwd_heads")
     return out, lse, ws
 
 

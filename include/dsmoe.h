@@ -260,8 +260,9 @@ const char* dsmoe_timing_stage_name(int stage);
  * is_causal (models/mla_triton.py:159-161) and no mask otherwise.  R, D_nope,
  * D_rope, D_v <= 256 as the reference requires (:186-196: DSMOE_ERR_INVALID),
  * and D_nope + D_rope <= 256 (DSMOE_ERR_UNSUPPORTED).  The workspace holds the
- * materialised K and V of every (batch, head): B * H * pad64(S_kv) *
- * (DQKp + DVp) * 2 + 256 bytes, DQKp = 2 D_nope + D_rope (D_nope + D_rope when
+ * materialised K and V of every (batch, head), B * H * pad64(S_kv) *
+ * (DQKp + DVp) * 2 bytes, and for calls of few query blocks the partial results
+ * of their key ranges (at most 512 blocks of 128 queries, fp32): DQKp = 2 D_nope + D_rope (D_nope + D_rope when
  * that exceeds 256) and DVp = D_v, each rounded up to a multiple of 16 and 32
  * (dsmoe_mla_attn_workspace_size gives the figure; about 2.7 GB at B 1,
  * H 128, S_kv 32768, D_nope 128, D_rope 64, D_v 128).  Row indices are 32-bit:
@@ -291,6 +292,13 @@ int dsmoe_mla_attn_fwd(const void* q_nope, const void* q_pe, const void* ctx_kv,
 int dsmoe_mla_attn_fwd_lse(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
                            const void* wkv_b_k, const void* wkv_b_v, const dsmoe_mla_dims* dims, void* out,
                            float* lse, void* workspace, size_t workspace_bytes, void* stream);
+/* Either of the two (lse NULL or not) with weights whose heads are D_nope (D_v)
+ * rows of R contiguous elements, wk_head_stride (wv_head_stride) elements apart:
+ * the per-head views of one wkv_b weight, read in place. */
+int dsmoe_mla_attn_fwd_heads(const void* q_nope, const void* q_pe, const void* ctx_kv, const void* ctx_pe,
+                             const void* wkv_b_k, int64_t wk_head_stride, const void* wkv_b_v, int64_t wv_head_stride,
+                             const dsmoe_mla_dims* dims, void* out, float* lse, void* workspace,
+                             size_t workspace_bytes, void* stream);
 /* The same attention for a few queries over a long cache (decoding): the query
  * is taken to the latent rows (q_nope W_k . ctx_kv) and the attention runs on
  * them, so no K and V are built; ranges of keys run side by side and are added

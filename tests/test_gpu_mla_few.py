@@ -62,6 +62,38 @@ def test_head_views_and_unaligned_rows():
     assert torch.equal(a, b) and torch.equal(a, c)
 
 
+@pytest.mark.parametrize("B,H,S_q,S_kv,R,Dn,Dr,Dv,causal,q_start", [
+    (1, 2, 200, 257, 64, 32, 16, 32, True, 57),        # two ranges
+    (1, 1, 70, 1500, 32, 16, 8, 10, True, 1200),       # as many ranges as there may be, element stores
+    (2, 3, 33, 700, 48, 24, 8, 40, True, 0),           # ranges past every query's position
+    (1, 2, 130, 400, 64, 32, 16, 96, False, 0),
+])
+def test_key_ranges(B, H, S_q, S_kv, R, Dn, Dr, Dv, causal, q_start):
+    """mla_fa_kernel over ranges of keys (few query blocks) and their sum, with the log-sum-exp; head views of one
+    weight and a workspace without room for the ranges."""
+    import dsmoe._lib as L
+    import dsmoe.mla as M
+    ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=S_q)
+    assert not M._few(S_q, R, Dn, Dv)
+    w = torch.cat([ts[4], ts[5]], 1)
+    ins, bc = M._prepare(*ts[:4], w[:, :Dn], w[:, Dn:])
+    out, lse, ws = M._forward(ins, bc, sc, causal, q_start, want_lse=True)
+    d = M._dims(ts[0], ts[1], ts[2], ts[5], sc, causal, q_start)
+    kv = 2 * B * H * (-(-S_kv // 64) * 64)
+    one = torch.empty_like(out)
+    lse1 = torch.empty_like(lse)
+    DQKp = next(16 * n for n in (2, 4, 6, 8, 12, 16) if 2 * Dn + Dr <= 16 * n)
+    DVp = next(32 * n for n in (1, 2, 4, 8) if Dv <= 32 * n)
+    small = -(-kv * (DQKp + DVp) // 256) * 256 + 256
+    assert small < int(L.load().dsmoe_mla_attn_workspace_size(d))
+    L.check(L.load().dsmoe_mla_attn_fwd_lse(*[L.ptr(t) for t in ts], d, L.ptr(one), L.ptr(lse1), L.ptr(ws), small,
+                                            L.stream_ptr(DEV)), "dsmoe_mla_attn_fwd_lse")
+    torch.cuda.synchronize()
+    _check(out, ts, sc, causal, q_start)
+    _check(one, ts, sc, causal, q_start)
+    torch.testing.assert_close(lse, lse1, rtol=1e-5, atol=1e-4)
+
+
 def test_gradients():
     """The backward builds K and V itself; it takes the log-sum-exp of this forward."""
     B, H, S_q, S_kv, R, Dn, Dr, Dv = 2, 3, 3, 70, 32, 16, 8, 24
