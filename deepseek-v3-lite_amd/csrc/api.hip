@@ -361,18 +361,43 @@ int dsmoe_permute_noalloc(const int32_t* idx, const dsmoe_dims* dims, int32_t* o
 //   E 16, D 1024, I 512, k 4 (64 tiles of 256 columns, rows per expert 25 / 50 / 83):
 //     gate/up 22 / 27 / 29 against 19 / 23 / 30, down 22 / 28 / 29 against 18 / 19 / 20;
 //   E 20, D 768, I 384, k 4 (60 tiles; 20 / 40 / 67 / 102 rows):
-//     gate/up 18 / 24 / 25 / 25 against 16 / 18 / 20 / 26, down 15 / 19 / 20 / 20 against 12 / 13 / 14 / 21;
-//   E 64, D 2048, I 1408, k 6, down (512 tiles and 16 long ones, a third round of
-//     CUs nearly empty; 9 / 19 / 31 / 48 rows): 122 / 137 / 142 / 143 against 91 / 105 / 121 / 141;
-//   the same, gate/up (704 tiles: 2.75 rounds, 5 TB/s): 143 / 146 / 150 / 154 against 164 / 194 / 225 / 257.
+//     gate/up 18 / 24 / 25 / 25 against 16 / 18 / 20 / 26, down 15 / 19 / 20 / 20 against 12 / 13 / 14 / 21.
+// With a CU's tile or more (E 64, D 2048: 704 gate/up tiles, 512 down tiles) it is the
+// slower one from 19 rows on: it reads the activations again for every 64 columns.
 constexpr int SK_MAX_T = SK_BM;
 
 static bool few_rows(int64_t rows, int groups, int n) {
-  const int64_t tiles = cdiv(n, 256) * groups;
-  if (tiles < 256) return rows <= 64 * (int64_t)groups;
-  // a last round of CUs less than a quarter full: the long tail costs more than re-read activations
-  const int64_t last = tiles % 256;
-  return last < 64 && tiles < 1024 && rows <= 40 * (int64_t)groups;
+  return cdiv(n, 256) * groups < 256 && rows <= 64 * (int64_t)groups;
+}
+
+// Tiles of 128 rows (launch_small of gemm.hip) or the persistent kernel's of 256:
+// whether the small ones are faster for `rows` routed rows over `groups` experts with
+// n output columns (SwiGLU: I), and dense_groups dense problems of dense_rows rows and
+// dense_n columns in the same launch.  Two lines, by tile counts:
+//  * The small tiles fit the GPU at once (one for each CU with the two accumulators of
+//    the SwiGLU, else two): a launch then lasts as long as one tile, and 256-row tiles
+//    leave most CUs idle.  Measured, whole forward in a graph, persistent kernel /
+//    small gate/up / small down (us; their tile counts): E 16, D 1024, I 512, S 1: T 300
+//    79 / 74 (184) / 71 (160), T 600 81 / 80 (272) / 74 (256), T 1200 83 / 99 (440) /
+//    77 (440), T 1500 85 / 103 / 84 (528), T 2048 89 / 108 / 89 (704); operator seam of
+//    3000 even rows 63 / 57 (248) / 55 (248), 8192 rows 66 / 82 (576) / 72 (576).
+//  * Store only: the 256-row tiles need a last round of CUs that is less than a quarter
+//    full (the dense tiles beside whole rounds of experts), and experts have up to 112
+//    rows, one small tile each.  E 64, D 2048, I 1408, S 2 (512 + 8 .. 40 tiles; rows per
+//    expert): T 65 (6) 268 us either way, T 200 (19) few-row kernel 290, small 271, T 333
+//    (31) 311, 280, T 450 (42) persistent 331, small 286, T 800 (75) 380, 339, T 1150
+//    (108) 376, 348, T 1300 (122) 365 both, T 1450 369, 384.  Without dense tiles (whole rounds)
+//    the persistent kernel is as fast: 400 rows 283 and few-row 285, 1200 rows 269 and 294.
+static bool small_tiles(int epi, int64_t rows, int groups, int n, int64_t dense_rows, int dense_groups, int dense_n) {
+  const bool swiglu = epi == EPI_SWIGLU;
+  const int64_t bn = swiglu ? 64 : 128;
+  // an expert's last tile is half full on average
+  const int64_t tiles = (rows / 128 + cdiv(groups, 2)) * cdiv(n, bn) +
+                        cdiv(dense_rows, 128) * dense_groups * cdiv(dense_n, bn);
+  if (tiles <= (swiglu ? 256 : 512)) return true;
+  if (swiglu || rows > 112 * (int64_t)groups) return false;
+  const int64_t big = cdiv(n, 256) * groups + cdiv(dense_rows, 256) * dense_groups * cdiv(dense_n, 256);
+  return big > 256 && big < 1024 && big % 256 > 0 && big % 256 < 64;
 }
 
 static size_t grouped_ws(const dsmoe_dims& d, void* base, const void*** ptrs, int32_t** off32, MTile** sched,
@@ -429,6 +454,8 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g.sched_count = g2.sched_count = cnt;
   g.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(d.T, d.E, bm);
   g.bm = g2.bm = bm;
+  g.small_tiles = small_tiles(EPI_SWIGLU, d.T, d.E, d.I, 0, 0, 0);
+  g2.small_tiles = small_tiles(EPI_STORE, d.T, d.E, d.D, 0, 0, 0);
   if (mfr && few_rows(d.T, d.E, 2 * d.I) && gemm_sk_ok(g))
     rc = launch_gemm_sk(g, EPI_SWIGLU, nullptr, st);
   else
@@ -553,6 +580,8 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   g1.sched_count = g2.sched_count = L.ps.sched_count;
   g1.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm);
   g1.bm = g2.bm = bm;
+  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.T, d.S, d.I_s);
+  g2.small_tiles = small_tiles(EPI_STORE, N, d.E, d.D, d.T, d.S ? 1 : 0, d.D);
   // (c) gate/up + SwiGLU: routed rows gathered from x through sorted_token,
   // and the shared experts as S dense groups over all tokens (h_shared =
   // [h_0 | h_1 | ...]), in one launch when the persistent kernel takes both
@@ -991,6 +1020,7 @@ int dsmoe_grouped_swiglu_bwd(const void* x_sorted, const void* const* w1, const 
   // recompute g = X W1^T, u = X W3^T, h = silu(g) * u
   g1.B0 = B.w1; g1.B1 = B.w3; g1.C = B.h; g1.Gs = B.g; g1.Us = B.u;
   g1.sched = B.sched_f; g1.sched_count = B.cnt_f; g1.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm_f); g1.bm = bm_f;
+  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, 0, 0, 0);
   rc = launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, d.dtype == DSMOE_F32 ? mf : mfr, st);
   if (rc) return rc;
   const int32_t mbound = (int32_t)sched_bound(N, d.E, BWD_BM);

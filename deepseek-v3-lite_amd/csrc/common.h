@@ -103,6 +103,7 @@ struct GemmDesc {
   int32_t groups;             // number of groups (dense)
   int32_t m_tiles_bound;      // host upper bound of M tiles (grid sizing)
   int32_t bm;                 // rows per M tile (must equal the schedule's tile height)
+  int32_t small_tiles;        // MFMA problems: 128-row tiles (gemm.hip) in place of the persistent kernel's 256
   // A operand: rows of length K (K contiguous)
   const void* A;
   int64_t lda;

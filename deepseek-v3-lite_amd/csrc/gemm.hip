@@ -15,8 +15,8 @@
 //
 // Kernels (the default bf16 path is the persistent gemm_qp_kernel of
 // gemm_qp.hip, the fp32 path gemm_f32.hip; this file holds the register-staged
-// MFMA kernel for the bf16 shapes that gemm_qp does not take, the FMA fallback
-// and the dispatcher):
+// MFMA kernel for the bf16 shapes that gemm_qp does not take and, on smaller
+// tiles, for launches of few tiles, the FMA fallback and the dispatcher):
 //   gemm_mfma_kernel  bf16 on gfx950 v_mfma_f32_32x32x16_bf16.  Block =
 //                     WM x WN waves, each owning TM x TN 32x32 output tiles
 //                     (x2 for SwiGLU: the W1 and W3 tiles of the same columns
@@ -65,16 +65,25 @@ __device__ __forceinline__ void store_rows(bf16_t* __restrict__ s, int lr, int l
   for (int i = 0; i < N; ++i) *reinterpret_cast<u32x4_t*>(s + swz(lr + i * RSTEP, lc)) = r[i];
 }
 
+// One launch computes g0 alone (pair = 0), or g0 and the dense problem g1 side by
+// side (pair = 1); row_scale applies to g0's rows only.
 template <int EPI, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const GemmDesc g, const float* __restrict__ row_scale) {
+__global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(const GemmDesc g0, const GemmDesc g1, const int pair,
+                                                                 const float* __restrict__ row_scale_0) {
   using CF = MfCfg<EPI, WM, WN, TM, TN>;
   constexpr int NB = CF::NB, BM = CF::BM, BN = CF::BN, RSTEP = CF::RSTEP;
   constexpr int A_LD = CF::A_LD, B_LD = CF::B_LD;
   extern __shared__ __attribute__((aligned(16))) bf16_t smem_mf[];
 
-  const int n_tiles = (int)cdiv(g.N, BN);
-  int grp, row0, rows, n_tile;
-  if (!tile_for_block<BM>(g, n_tiles, grp, row0, rows, n_tile)) return;
+  int which = 0, grp, row0, rows, n_tile;
+  if (pair) {
+    if (!tile_for_block_pair<BM>(g0, g1, BN, which, grp, row0, rows, n_tile)) return;
+    which = __builtin_amdgcn_readfirstlane(which);
+  } else {
+    if (!tile_for_block<BM>(g0, (int)cdiv(g0.N, BN), grp, row0, rows, n_tile)) return;
+  }
+  const GemmDesc& g = which ? g1 : g0;
+  const float* __restrict__ row_scale = which ? nullptr : row_scale_0;
   const int n0 = n_tile * BN;
 
   const int tid = threadIdx.x;
@@ -314,7 +323,8 @@ static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // MFMA kernels use 256-row M tiles (the routed schedule height): the
 // persistent eight-wave kernel of gemm_qp.hip (K slabs of 64 streamed by
-// direct loads) wherever its constraints hold, else gemm_mfma_kernel with 8
+// direct loads) wherever its constraints hold (128-row tiles of gemm_mfma_kernel
+// where those are faster, launch_small), else gemm_mfma_kernel with 8
 // waves (4 x 2), per wave 2 x 2 tiles (SwiGLU: x2) or 2 x 4 (store).
 constexpr int MF_BM = 256;
 
@@ -331,24 +341,41 @@ bool gemm_mfma_eligible(const GemmDesc& g, int dtype, bool allow_mfma) {
 
 int gemm_tile_m(bool mfma) { return mfma ? MF_BM : TILE_M; }
 
-static int64_t grid_for(const GemmDesc& g, int bm, int tile_n) {
-  const int64_t m_bound = g.sched ? g.m_tiles_bound : cdiv(g.dense_rows, bm) * g.groups;
-  const int64_t total = m_bound * cdiv(g.N, tile_n);
-  return 8 * cdiv(total, 8);
+// M tiles of height bm that the grid has to cover (a schedule of height g.bm is
+// cut into g.bm / bm tiles an entry).
+static int64_t m_tiles_for(const GemmDesc& g, int bm) {
+  return g.sched ? (int64_t)g.m_tiles_bound * (g.bm / bm) : cdiv(g.dense_rows, bm) * g.groups;
 }
 
+static int64_t grid_for(const GemmDesc& g, int bm, int tile_n) {
+  return 8 * cdiv(m_tiles_for(g, bm) * cdiv(g.N, tile_n), 8);
+}
+
+// g1: a dense problem for the same launch, or null.
 template <int EPI, int WM, int WN, int TM, int TN>
-static int launch_mfma_t(const GemmDesc& g, const float* row_scale, hipStream_t st) {
+static int launch_mfma_t(const GemmDesc& g, const GemmDesc* g1, const float* row_scale, hipStream_t st) {
   using CF = MfCfg<EPI, WM, WN, TM, TN>;
-  static_assert(CF::BM == MF_BM, "schedule height");
-  const int64_t grid = grid_for(g, CF::BM, CF::BN);
+  static_assert(MF_BM % CF::BM == 0, "schedule height");
+  int64_t grid = grid_for(g, CF::BM, CF::BN);
+  if (g1) grid += grid_for(*g1, CF::BM, CF::BN);
   if (grid == 0) return DSMOE_OK;
   auto kern = gemm_mfma_kernel<EPI, WM, WN, TM, TN>;
   static const hipError_t attr =
       hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CF::LDS_BYTES);
   if (attr != hipSuccess) return fail(DSMOE_ERR_HIP, "gemm: cannot raise LDS limit");
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(CF::THREADS), CF::LDS_BYTES, st, g, row_scale);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(CF::THREADS), CF::LDS_BYTES, st, g, g1 ? *g1 : g, g1 ? 1 : 0,
+                     row_scale);
   return check_launch("gemm_mfma");
+}
+
+// The 128-row tiles: 4 waves, 64 KB of LDS (two blocks a CU), 128 columns (SwiGLU: 64 of
+// h).  For launches whose 256-row tiles would leave CUs idle (GemmDesc.small_tiles;
+// the line and both sides' times stand at small_tiles() of api.hip).  What bounds a
+// tile there is the latency of its K / 64 slabs, not the matrix cores; fetching two or
+// four slabs ahead into registers was slower (both GEMMs of 1200 rows, E 16, D 1024: 49 -> 64 and 61 us).
+static int launch_small(const GemmDesc& g, const GemmDesc* gd, int epi, const float* row_scale, hipStream_t st) {
+  if (epi == EPI_SWIGLU) return launch_mfma_t<EPI_SWIGLU, 2, 2, 2, 1>(g, gd, row_scale, st);
+  return launch_mfma_t<EPI_STORE, 2, 2, 2, 2>(g, gd, row_scale, st);
 }
 
 int launch_grouped_gemm(const GemmDesc& g_in, int epi, int dtype, const float* row_scale, bool allow_mfma,
@@ -358,11 +385,12 @@ int launch_grouped_gemm(const GemmDesc& g_in, int epi, int dtype, const float* r
   if (dtype == DSMOE_F32) return launch_gemm_f32(g, nullptr, epi, row_scale, allow_mfma, st);
   if (gemm_mfma_eligible(g, dtype, allow_mfma)) {
     if (g.bm != MF_BM) return fail(DSMOE_ERR_INVALID, "gemm: schedule tile height does not match the MFMA kernel");
-    if (gemm_qp_ok(g)) return launch_gemm_qp(g, epi, row_scale, st);
+    if (gemm_qp_ok(g))
+      return g.small_tiles ? launch_small(g, nullptr, epi, row_scale, st) : launch_gemm_qp(g, epi, row_scale, st);
     // shapes the persistent kernel does not take (N % 8 == 4, more than two K
     // segments, 8-byte aligned output): the register-staged 8-wave kernel
-    if (epi == EPI_SWIGLU) return launch_mfma_t<EPI_SWIGLU, 4, 2, 2, 2>(g, row_scale, st);
-    return launch_mfma_t<EPI_STORE, 4, 2, 2, 4>(g, row_scale, st);
+    if (epi == EPI_SWIGLU) return launch_mfma_t<EPI_SWIGLU, 4, 2, 2, 2>(g, nullptr, row_scale, st);
+    return launch_mfma_t<EPI_STORE, 4, 2, 2, 4>(g, nullptr, row_scale, st);
   }
   if (g.bm != TILE_M) return fail(DSMOE_ERR_INVALID, "gemm: schedule tile height does not match the SIMT kernel");
   const int64_t grid = grid_for(g, TILE_M, SM_N);
@@ -382,7 +410,8 @@ int launch_grouped_gemm_pair(const GemmDesc& gr_in, const GemmDesc& gd_in, int e
   const bool one = gd.sched == nullptr && gr.N > 0 && gr.K > 0 && gd.N > 0 &&
                    gd.K > 0 && gemm_mfma_eligible(gr, dtype, allow_mfma_r) && gemm_mfma_eligible(gd, dtype, allow_mfma_d) &&
                    gemm_qp_ok(gr) && gemm_qp_ok(gd);
-  if (one) return launch_gemm_qp_pair(gr, gd, epi, row_scale, st);
+  if (one)
+    return gr.small_tiles ? launch_small(gr, &gd, epi, row_scale, st) : launch_gemm_qp_pair(gr, gd, epi, row_scale, st);
   const int rc = launch_grouped_gemm(gr_in, epi, dtype, row_scale, allow_mfma_r, st);
   if (rc) return rc;
   return launch_grouped_gemm(gd_in, epi, dtype, nullptr, allow_mfma_d, st);

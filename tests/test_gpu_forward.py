@@ -487,3 +487,18 @@ def test_few_rows_per_expert(case, skew, training):
         assert counts.tolist() == [0, case.T, 0, 0]
     ref = R.moe_forward_ref(x, p, case.k, indices=idx.cpu())
     torch.testing.assert_close(y.cpu().float(), ref.float(), rtol=2e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("case,skew", [
+    (CS.Case("small_both", 300, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False),   # about 75 rows each
+    (CS.Case("small_edges", 200, 320, 2, 192, 2, 2, 64, torch.bfloat16), False),   # partial N tile, 200 = 128 + 72 rows
+    (CS.Case("small_skew", 390, 256, 4, 128, 1, 1, 192, torch.bfloat16), True),    # one expert with every row: 3 x 128 + 6
+    (CS.Case("small_alone", 513, 256, 8, 128, 3, 0, 0, torch.bfloat16, "normal"), False),   # no shared expert
+    (CS.Case("small_tail", 130, 2048, 64, 128, 4, 1, 128, torch.bfloat16, "normal"), False),   # down: 512 + 8 big tiles
+    (CS.Case("past_small", 2050, 1088, 12, 320, 4, 2, 192, torch.bfloat16, "normal"), False),  # the persistent kernel
+], ids=lambda c: str(c) if isinstance(c, bool) else f"{c.name}_T{c.T}")
+def test_small_tiles(case, skew, training):
+    """Launches of few tiles on 128-row tiles, routed and shared experts in one launch; past the line the persistent
+    kernel with partial tiles."""
+    test_few_rows_per_expert(case, skew, training)
