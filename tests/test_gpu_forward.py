@@ -469,11 +469,11 @@ def test_update_bias_with_fractional_counts():
     (CS.Case("few_unfilled", 65, 256, 16, 128, 2, 1, 128, torch.bfloat16, "normal"), False),   # both GEMMs few-row
     (CS.Case("few_unfilled", 190, 256, 4, 256, 1, 1, 128, torch.bfloat16), True),   # one expert with every row: 64-row parts
     (CS.Case("few_unfilled", 256, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False),  # at the line: 64 rows each
-    (CS.Case("few_down", 70, 2048, 64, 256, 4, 2, 256, torch.bfloat16, "normal"), False),   # the down projection alone
+    (CS.Case("few_down", 70, 2048, 64, 256, 4, 2, 256, torch.bfloat16, "normal"), False),   # gate/up alone, down on 128-row tiles
 ], ids=lambda c: str(c) if isinstance(c, bool) else f"{c.name}_T{c.T}")
 def test_few_rows_per_expert(case, skew, training):
     """More than 64 tokens with few rows per expert: the few-row GEMM on schedules of its own height and of 256 rows,
-    beside the persistent one."""
+    beside the other kernels."""
     x, p, _ = CS.make_inputs(case)
     if skew:
         p = R.MoEParams(p.gate_w, torch.tensor([0.0, 5.0, 0.0, 0.0]), p.w1, p.w2, p.w3, p.sw1, p.sw2, p.sw3)
