@@ -72,6 +72,11 @@ __device__ __forceinline__ bf16x8_t few_ld8(const bf16_t* p, int n, bool vec) {
   return __builtin_bit_cast(bf16x8_t, v);
 }
 
+// The first key that no row of tile mt sees (at least 1).
+__device__ __forceinline__ int few_kend(const MlaFew& a, int mt) {
+  return a.causal ? min(a.S_kv, (min(a.M, 32 * mt + 32) - 1) / a.H + a.q_start + 1) : a.S_kv;
+}
+
 // Grid (M, B).  Thread (g, c): columns 8 c .. 8 c + 7 over the D_nope rows g,
 // g + groups, ..., the groups added through LDS.
 __global__ __launch_bounds__(256) void mla_absorb_kernel(const MlaFew a) {
@@ -113,7 +118,8 @@ __global__ __launch_bounds__(256) void mla_absorb_kernel(const MlaFew a) {
     dst[2 * a.Rq + d] = d < a.Dr ? (bf16_t)(qp[d] ^ (a.neg ? 0x8000 : 0)) : bf16_t(0);
 }
 
-// One wave per (batch, row tile, key range), range fastest.  NS = Rq / 16; VEC:
+// One wave per (batch, row tile, key range), range fastest.  A range past few_kend
+// writes nothing (mla_few_out_kernel does not read it).  NS = Rq / 16; VEC:
 // 16-byte loads of latent and rope rows.
 template <int NS, bool VEC>
 __global__ __launch_bounds__(256) void mla_few_kernel(const MlaFew a) {
@@ -129,14 +135,9 @@ __global__ __launch_bounds__(256) void mla_few_kernel(const MlaFew a) {
   if (b >= a.B) return;
   const int row = 32 * mt + l32;
   const int qpos = row / a.H + a.q_start;
-  int kend = a.S_kv;
-  if (a.causal) kend = min(kend, (min(a.M, 32 * mt + 32) - 1) / a.H + a.q_start + 1);
-  const int kb = split * a.cpw * 32, ke = min(kend, kb + a.cpw * 32);
+  const int kb = split * a.cpw * 32, ke = min(few_kend(a, mt), kb + a.cpw * 32);
   const int64_t part = ((int64_t)b * a.nsplit + split) * a.Mp + row;
-  if (kb >= ke) {
-    if (hi == 0 && row < a.M) a.ml[part] = make_float2(-INFINITY, 0.0f);
-    return;
-  }
+  if (kb >= ke) return;
   char* tile = few_tile + wave * 32 * RB;
   const MlbLane<RB> lk(lane);
   const bf16_t* qrow = a.qabs + ((int64_t)b * a.Mp + min(row, a.M - 1)) * (2 * a.Rq + a.Drp) + 8 * hi;
@@ -241,6 +242,10 @@ __global__ __launch_bounds__(256) void mla_few_kernel(const MlaFew a) {
           make_float4(o[v][4 * g], o[v][4 * g + 1], o[v][4 * g + 2], o[v][4 * g + 3]);
 }
 
+// The ranges of a row added by their weights.  Every range that mla_few_kernel
+// wrote takes part, whatever it holds: a NaN in one key, or in the query, reaches
+// the sum as in mla.hip, also through a weight of 0 (a range whose scores are all
+// NaN has no maximum).
 // Grid (M, B).  LDS (floats): weights of the ranges [FEW_MAX_SPLITS] | group sums
 // [groups][Rq] (the first row then holds the normalised sum).
 __global__ __launch_bounds__(256) void mla_few_out_kernel(const MlaFew a) {
@@ -250,6 +255,7 @@ __global__ __launch_bounds__(256) void mla_few_out_kernel(const MlaFew a) {
   const int tid = threadIdx.x, row = blockIdx.x, b = blockIdx.y;
   const int s = row / a.H, h = row - s * a.H;
   const int64_t p0 = (int64_t)b * a.nsplit * a.Mp + row;
+  const int nr = min(a.nsplit, (few_kend(a, row / 32) + 32 * a.cpw - 1) / (32 * a.cpw));   // ranges written
   // every wave reduces the ranges' maxima and normalisers, two ranges per lane
   const int lane = tid & 63;
   static_assert(FEW_MAX_SPLITS == 128, "two ranges per lane");
@@ -257,8 +263,8 @@ __global__ __launch_bounds__(256) void mla_few_out_kernel(const MlaFew a) {
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int i = lane + 64 * u;
-    r2[u] = a.ml[p0 + (int64_t)min(i, a.nsplit - 1) * a.Mp];
-    if (i >= a.nsplit) r2[u] = make_float2(-INFINITY, 0.0f);
+    r2[u] = a.ml[p0 + (int64_t)min(i, nr - 1) * a.Mp];
+    if (i >= nr) r2[u] = make_float2(-INFINITY, 0.0f);
   }
   float m = fmaxf(r2[0].x, r2[1].x);
 #pragma unroll
@@ -266,7 +272,7 @@ __global__ __launch_bounds__(256) void mla_few_out_kernel(const MlaFew a) {
   float lt = 0.0f;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const float w = r2[u].y > 0.0f ? __builtin_amdgcn_exp2f((r2[u].x - m) * a.c) : 0.0f;
+    const float w = r2[u].x != -INFINITY ? __builtin_amdgcn_exp2f((r2[u].x - m) * a.c) : 0.0f;
     lt = fmaf(w, r2[u].y, lt);
     if (tid < 64) wt[lane + 64 * u] = w;
   }
@@ -280,16 +286,16 @@ __global__ __launch_bounds__(256) void mla_few_out_kernel(const MlaFew a) {
     const float* po = a.po + p0 * a.Rq + 4 * c;
     const int64_t step = (int64_t)a.Mp * a.Rq;
     constexpr int U = 6;   // loads in flight
-    for (int i = g; i < a.nsplit; i += U * groups) {
+    for (int i = g; i < nr; i += U * groups) {
       float4 v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        v[u] = *reinterpret_cast<const float4*>(po + min(i + u * groups, a.nsplit - 1) * step);
+        v[u] = *reinterpret_cast<const float4*>(po + min(i + u * groups, nr - 1) * step);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float w = i + u * groups < a.nsplit ? wt[min(i + u * groups, FEW_MAX_SPLITS - 1)] : 0.0f;
-        const bool on = w > 0.0f;   // a range without a visible key wrote no sums
+        const bool on = i + u * groups < nr;
+        const float w = wt[min(i + u * groups, FEW_MAX_SPLITS - 1)];
         acc.x = fmaf(w, on ? v[u].x : 0.0f, acc.x);
         acc.y = fmaf(w, on ? v[u].y : 0.0f, acc.y);
         acc.z = fmaf(w, on ? v[u].z : 0.0f, acc.z);

@@ -48,6 +48,24 @@ def test_scales(scale):
     _check(_run(ts, scale, True, 150), ts, scale, True, 150)
 
 
+@pytest.mark.parametrize("S_q,causal", [(1, True), (3, False), (70, False)])   # latent rows twice, K and V in two ranges
+def test_nan_reaches_the_rows_that_see_it(S_q, causal):
+    """A NaN in a latent row, a rope row or a query: NaN in every output that depends on it, whatever the other key
+    ranges hold, and no other output changed."""
+    from dsmoe.mla import mla_attention
+    B, H, S_kv = 2, 3, 300
+    ts, sc = _inputs(B, H, S_q, S_kv, 64, 32, 16, 24, seed=6)
+    call = lambda ins: mla_attention(*ins, sc, is_causal=causal, q_start=S_kv - 1)
+    clean = call(ts)
+    for which, at, rows in ((2, (1, 77, 5), 1), (3, (0, 299, 0), 0), (0, (0, 2, S_q - 1, 3), (0, S_q - 1, 2)),
+                            (1, (1, 1, 0, 0), (1, 0, 1))):
+        bad = [t.clone() for t in ts]
+        bad[which][at] = float("nan")
+        want = clean.clone()
+        want[rows] = float("nan")
+        torch.testing.assert_close(call(bad), want, rtol=0, atol=0, equal_nan=True)
+
+
 def test_head_views_and_unaligned_rows():
     """The per-head views of one weight, and latent rows two bytes past a 16-byte boundary: the aligned call's
     result, bit for bit (the same values in the same order)."""
