@@ -13,8 +13,9 @@
 // work and the W traffic per workgroup shrink with ks.  With ks splits the
 // partial logits go to a workspace and the routing launch adds them in split
 // order; without a workspace (ks = 1) the workgroup routes its own tokens.
-// fp32 x in the layer: fp32 MFMA partial logits (gate_f32_kernel) and the same
-// routing launch.  Other shapes, and fp32 x without a workspace: SIMT FMA tiles.
+// fp32 x: fp32 MFMA partial logits (gate_f32_kernel) and the same routing
+// launch; without a workspace one launch adds the same partial logits in the same
+// order and routes (gate_f32_route_kernel).  Other shapes: SIMT FMA tiles.
 //
 // Routing.  One wave per token, one lane per expert (E <= 64; E <= 256 with
 // several experts per lane): sigmoid in double rounded once, + bias, then k
@@ -364,26 +365,21 @@ __global__ __launch_bounds__(RR_WAVES * 64) void route_rank_kernel(const float* 
 
 // ------------------------------------------------------------------ fp32 MFMA logits (fp32 x)
 // A wave takes 32 tokens, every expert (NT tiles of 32) and one of ks ranges of
-// D / 8 column groups, and writes its partial logits; no LDS, no barrier.  Lane
-// half h of group g holds columns 8 g + 4 h .. + 3 of token (of x) and of expert
-// (of W) lane & 31, so one 16-byte load of each feeds four v_mfma_f32_32x32x2_f32.
+// D / 8 column groups; no LDS, no barrier.  Lane half h of group g holds columns
+// 8 g + 4 h .. + 3 of token (of x) and of expert (of W) lane & 31, so one 16-byte
+// load of each feeds four v_mfma_f32_32x32x2_f32.
 // Bound by latency: at T 2048, D 768, E 20 it reads 6.3 MB of x once, and W (61 KB)
-// from L2 for every token tile.  The FMA tiles it replaces in the layer put 128
+// from L2 for every token tile.  The FMA tiles it replaces put 128
 // tokens on a workgroup (16 workgroups at T 2048) and walked D in 32-column
 // chunks, one memory latency and two barriers each: 212 us there, 39 us at T 1024, D 64.
 constexpr int GF_TOK = 32;
 
+// Partial logits of tokens t0 .. t0 + 31 over range `split`: lane holds token
+// lane & 31 and, per q, experts 32 i + 8 q + 4 (lane >> 5) + {0..3} in acc[i][4 q + ..].
 template <int NT>
-__global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__ x, const float* __restrict__ gw, int T,
-                                                       int D, int E, float* __restrict__ part, int ks,
-                                                       const PtrChunk tables, const void** tab_dst) {
-  const int tid = threadIdx.x, lane = tid & 63;
-  if (blockIdx.x == 0)
-    for (int i = tid; i < tables.n; i += blockDim.x) tab_dst[tables.off + i] = tables.p[i];
-  const int64_t unit = (int64_t)blockIdx.x * 4 + (tid >> 6);   // (token tile, split), split fastest
-  const int split = (int)(unit % ks);
-  const int64_t t0 = unit / ks * GF_TOK;
-  if (t0 >= T) return;
+__device__ __forceinline__ void gate_f32_part(const float* __restrict__ x, const float* __restrict__ gw, int64_t t0,
+                                              int T, int D, int E, int split, int ks, g_f32x16_t (&acc)[NT]) {
+  const int lane = threadIdx.x & 63;
   const int groups = (D + 7) / 8, per = (groups + ks - 1) / ks;
   const int g0 = split * per, g1 = min(groups, g0 + per);
   const int m = lane & 31, kh = 4 * (lane >> 5);
@@ -391,7 +387,6 @@ __global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__
   const float* wr[NT];
 #pragma unroll
   for (int i = 0; i < NT; ++i) wr[i] = gw + (int64_t)min(32 * i + m, E - 1) * D;
-  g_f32x16_t acc[NT] = {};
   constexpr int U = NT <= 2 ? 6 : NT <= 4 ? 4 : 2;   // groups in flight; groups past the range count as zeros
   for (int g = g0; g < g1; g += U) {
     g_f32x4_t xv[U], wv[U][NT];
@@ -413,7 +408,24 @@ __global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__
           acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? wv[u][i][q] : 0.0f, in ? xv[u][q] : 0.0f, acc[i], 0, 0, 0);
     }
   }
-  // lane holds token m and, per q, experts 32 i + 8 q + 4 (lane >> 5) + {0..3}
+}
+
+// Partial logits to part[(split * T + t) * E + e]; unit (token tile, split) per
+// wave, split fastest.
+template <int NT>
+__global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__ x, const float* __restrict__ gw, int T,
+                                                       int D, int E, float* __restrict__ part, int ks,
+                                                       const PtrChunk tables, const void** tab_dst) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (blockIdx.x == 0)
+    for (int i = tid; i < tables.n; i += blockDim.x) tab_dst[tables.off + i] = tables.p[i];
+  const int64_t unit = (int64_t)blockIdx.x * 4 + (tid >> 6);
+  const int split = (int)(unit % ks);
+  const int64_t t0 = unit / ks * GF_TOK;
+  if (t0 >= T) return;
+  g_f32x16_t acc[NT] = {};
+  gate_f32_part<NT>(x, gw, t0, T, D, E, split, ks, acc);
+  const int m = lane & 31, kh = 4 * (lane >> 5);
   if (t0 + m >= T) return;
   float* pr = part + ((int64_t)split * T + t0 + m) * E;
 #pragma unroll
@@ -431,6 +443,55 @@ __global__ __launch_bounds__(256) void gate_f32_kernel(const float* __restrict__
           if (e + r < E) pr[e + r] = acc[i][4 * q + r];
       }
     }
+}
+
+// The gate on its own (no workspace): a workgroup takes 32 tokens, wave w range w,
+// the ranges are added in LDS in the order of the routing launch, and the
+// workgroup routes: the layer's logits bit for bit, so both take the same experts.
+// T 2048, D 768, E 20, in a graph with the fill of the counts: 17 us (FMA tiles 145).
+// LDS (4-byte words): lg[32][E + 1] | bias[E] | hist[E] | routing scratch [64 per wave]
+template <int NT>
+__global__ __launch_bounds__(64 * GATE_KS_MAX) void gate_f32_route_kernel(const float* __restrict__ x,
+                                                                          const float* __restrict__ gw,
+                                                                          const float* __restrict__ bias, int T, int D,
+                                                                          int E, int k, float route_scale, GateOut out,
+                                                                          int ks) {
+  extern __shared__ __attribute__((aligned(16))) float rsm[];
+  const int ldl = E + 1;
+  float* lg = rsm;
+  float* bias_s = lg + GF_TOK * ldl;
+  int32_t* hist = reinterpret_cast<int32_t*>(bias_s + E);
+  int32_t* scr = hist + E;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t0 = blockIdx.x * GF_TOK;
+  for (int e = tid; e < E; e += blockDim.x) {
+    bias_s[e] = bias[e];
+    hist[e] = 0;
+  }
+  g_f32x16_t acc[NT] = {};
+  if (wave < ks) gate_f32_part<NT>(x, gw, t0, T, D, E, wave, ks, acc);
+  float* pl = lg + (lane & 31) * ldl + 4 * (lane >> 5);
+  for (int sp = 0; sp < ks; ++sp) {
+    if (wave == sp) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = 32 * i + 8 * (r >> 2) + (r & 3);
+          if (c + 4 * (lane >> 5) < E) pl[c] = sp ? pl[c] + acc[i][r] : acc[i][r];
+        }
+    }
+    __syncthreads();
+  }
+  const int ntok = min(GF_TOK, T - t0);
+  if (out.logits)
+    for (int i = tid; i < ntok * E; i += blockDim.x) {
+      const int t = i / E, e = i - t * E;
+      out.logits[(int64_t)(t0 + t) * E + e] = lg[t * ldl + e];
+    }
+  route_tokens(lg, ldl, ntok, t0, bias_s, E, k, route_scale, DSMOE_F32, out, out.counts ? hist : nullptr, nullptr, scr);
+  __syncthreads();
+  flush_hist(hist, E, out.counts);
 }
 
 // ------------------------------------------------------------------ SIMT logits (other shapes)
@@ -652,6 +713,14 @@ static int launch_gate_f32(const void* x, const float* gw, const float* bias, co
   none.n = 0;
   none.off = 0;
   const int ks = gate_k_splits(d);
+  if (!part) {
+    auto kern = d.E <= 32 ? gate_f32_route_kernel<1>
+                : d.E <= 64 ? gate_f32_route_kernel<2> : d.E <= 128 ? gate_f32_route_kernel<4> : gate_f32_route_kernel<8>;
+    const size_t lds = sizeof(float) * (GF_TOK * (d.E + 1) + 2 * d.E + 64 * GATE_KS_MAX);   // at most 37 KB
+    hipLaunchKernelGGL(kern, dim3((unsigned)cdiv(d.T, GF_TOK)), dim3(64 * GATE_KS_MAX), lds, st,
+                       static_cast<const float*>(x), gw, bias, d.T, d.D, d.E, d.k, d.route_scale, out, ks);
+    return check_launch("gate_f32_route");
+  }
   const unsigned blocks = (unsigned)cdiv(cdiv(d.T, GF_TOK) * ks, 4);
   auto kern = d.E <= 32 ? gate_f32_kernel<1>
               : d.E <= 64 ? gate_f32_kernel<2> : d.E <= 128 ? gate_f32_kernel<4> : gate_f32_kernel<8>;
@@ -682,7 +751,7 @@ int launch_gate(const void* x, const float* logits_in, const float* gw, const fl
       default: return launch_gate_mfma_nt<8>(x, gw, bias, d, out, part, tables, tab_dst, po, ranked, st);
     }
   }
-  if (part && gate_f32_ok(x, gw, d)) return launch_gate_f32(x, gw, bias, d, out, part, tables, tab_dst, po, ranked, st);
+  if (gate_f32_ok(x, gw, d)) return launch_gate_f32(x, gw, bias, d, out, part, tables, tab_dst, po, ranked, st);
   if (d.dtype == DSMOE_BF16) {
     if (d.E <= 16) return launch_gate_t<bf16_t, 16>(x, gw, bias, d, out, st);
     if (d.E <= 32) return launch_gate_t<bf16_t, 32>(x, gw, bias, d, out, st);

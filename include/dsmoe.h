@@ -74,6 +74,9 @@ int dsmoe_version(void);
  *   weights_x   (T,k) weights cast to x dtype (_last_weights), may be NULL
  *   sel_scores  (T,k) fp32 unbiased scores of the selected experts, may be NULL
  *   counts      (E)   int32 per-expert histogram (== bincount(idx)), may be NULL
+ * For fp32 x the logits are those of the gate inside dsmoe_moe_fwd bit for bit.
+ * For bf16 x that gate sums K ranges and this one does not, so logits can
+ * differ in the last bits, and a token at a near tie can take another expert.
  */
 int dsmoe_gate_fwd(const void* x, const float* gate_w, const float* gate_bias, const dsmoe_dims* dims,
                    float* logits, int32_t* idx, int64_t* idx64, float* weights, void* weights_x,

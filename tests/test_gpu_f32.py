@@ -9,6 +9,7 @@ import torch
 from oracle import moe_ref as R
 from tests import _cases as CS
 from tests.test_gpu_backward import _close, _run
+from tests.test_gpu_forward import _layer_raw
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +59,18 @@ def test_unaligned_weights_take_the_element_loads():
         b = moe_layer(shift(x), shift(gw), gb, *map(sh, (p.w1, p.w2, p.w3, p.sw1, p.sw2, p.sw3)), k=k)
     assert torch.equal(a[1], b[1])
     _close(a[0].cpu(), b[0].cpu(), 1e-5, 1e-5 * a[0].abs().max().item(), "y")
+
+
+@pytest.mark.parametrize("T,D,E,k", [(1, 64, 4, 2), (33, 8, 20, 4), (2048, 768, 20, 4), (300, 256, 40, 2), (65, 68, 97, 3),
+                                     (520, 132, 200, 2), (70, 2052, 130, 9), (96, 63, 3, 3)], ids=str)
+def test_the_gate_alone_equals_the_layers(T, D, E, k):
+    """dsmoe_gate_fwd and the gate inside dsmoe_moe_fwd on fp32 x: the same logits bit for bit, hence the same experts,
+    order and weights, near ties included."""
+    from dsmoe import ops
+    case = CS.Case("gate", T, D, E, 32, k, 0, 0, torch.float32, "normal", 1.5)
+    x, p, _ = CS.make_inputs(case)
+    dev = lambda t: t.to("cuda:0")
+    gate = ops.gate_forward(dev(x), dev(p.gate_w), dev(p.gate_bias), k, 1.5, want_logits=True)
+    layer = _layer_raw(case, x, p)
+    for name in ("logits", "idx", "weights", "counts"):
+        assert (gate[name].cpu().numpy() == layer[name]).all(), name
