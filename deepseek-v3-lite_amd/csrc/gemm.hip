@@ -348,7 +348,7 @@ static int64_t m_tiles_for(const GemmDesc& g, int bm) {
 }
 
 static int64_t grid_for(const GemmDesc& g, int bm, int tile_n) {
-  return 8 * cdiv(m_tiles_for(g, bm) * cdiv(g.N, tile_n), 8);
+  return tile_grid(m_tiles_for(g, bm), cdiv(g.N, tile_n), g.sched && g.bm != bm);
 }
 
 // g1: a dense problem for the same launch, or null.

@@ -203,8 +203,9 @@ bool gemm_sk_ok(const GemmDesc& g) {
          a16(g.A) && a16(g.C) && g.Gs == nullptr && g.Us == nullptr;
 }
 
-static int64_t sk_mtiles(const GemmDesc& g) {
-  return g.sched ? (int64_t)g.m_tiles_bound * (g.bm / SK_BM) : cdiv(g.dense_rows, SK_BM) * g.groups;
+static int64_t sk_grid(const GemmDesc& g, int bn) {
+  const int64_t m = g.sched ? (int64_t)g.m_tiles_bound * (g.bm / SK_BM) : cdiv(g.dense_rows, SK_BM) * g.groups;
+  return tile_grid(m, cdiv(g.N, bn), g.sched && g.bm != SK_BM);
 }
 
 template <int EPI>
@@ -218,15 +219,14 @@ static int sk_launch(const GemmDesc& g0, const GemmDesc& g1, int pair, const flo
 
 int launch_gemm_sk(const GemmDesc& g, int epi, const float* row_scale, hipStream_t st) {
   const int bn = (epi == EPI_SWIGLU) ? SKCfg<EPI_SWIGLU>::BN : SKCfg<EPI_STORE>::BN;
-  const int64_t grid = 8 * cdiv(sk_mtiles(g) * cdiv(g.N, bn), 8);
+  const int64_t grid = sk_grid(g, bn);
   return epi == EPI_SWIGLU ? sk_launch<EPI_SWIGLU>(g, g, 0, row_scale, grid, st)
                            : sk_launch<EPI_STORE>(g, g, 0, row_scale, grid, st);
 }
 
 int launch_gemm_sk_pair(const GemmDesc& gr, const GemmDesc& gd, int epi, const float* row_scale, hipStream_t st) {
   const int bn = (epi == EPI_SWIGLU) ? SKCfg<EPI_SWIGLU>::BN : SKCfg<EPI_STORE>::BN;
-  const int64_t td = sk_mtiles(gd) * cdiv(gd.N, bn), tr = sk_mtiles(gr) * cdiv(gr.N, bn);
-  const int64_t grid = 8 * (cdiv(td, 8) + cdiv(tr, 8));
+  const int64_t grid = sk_grid(gd, bn) + sk_grid(gr, bn);
   return epi == EPI_SWIGLU ? sk_launch<EPI_SWIGLU>(gr, gd, 1, row_scale, grid, st)
                            : sk_launch<EPI_STORE>(gr, gd, 1, row_scale, grid, st);
 }

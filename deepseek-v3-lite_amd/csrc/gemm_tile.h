@@ -5,19 +5,57 @@
 
 namespace dsmoe {
 
+// Tile j of XCD x of a routed schedule of height bm cut into sub = bm / BM parts an
+// entry.  Parts past an entry's rows are no work, and how many there are differs
+// between entries, so the parts are listed part by part (the first of every entry,
+// the second of every entry, ...; N fastest) and the list is dealt to the XCDs in
+// runs of CUT_RUN tiles: each XCD gets an eighth of the first parts, and surplus
+// blocks come last.  Measured (us; entry by entry in eighths of the list, then so):
+//   E 8, D 2048, I 1408, k 2, T 200, one expert with every token, 64-row tiles of the
+//   down projection on a 256-row schedule: 49, 28 (one XCD held the large expert alone);
+//   E 128, D 1024, I 128, k 1, T 512, 128-row gate/up tiles: 41, 26 (surplus blocks
+//   between the real ones left half of an XCD's CUs idle);
+//   E 64, D 2048, I 1408, k 6, T 1000, three experts with every token, 128-row down
+//   tiles: 181, 132; even routing 112, 111.
+// Whole parts in turn instead of runs leave XCDs idle where parts are few (E 2, D 4096,
+// I 4096, T 300: 64, 82; runs of 4: 61); runs of 1, 2 and 8 measure as runs of 4.
+constexpr int CUT_RUN = 4;
+
+template <int BM>
+__device__ __forceinline__ bool cut_tile(const GemmDesc& g, int sub, int n_tiles, int64_t j, int x, int& grp, int& row0,
+                                         int& rows, int& n_tile) {
+  const int entries = *g.sched_count;
+  const int64_t lin = (j / CUT_RUN * 8 + x) * CUT_RUN + j % CUT_RUN, part = lin / n_tiles;
+  n_tile = (int)(lin - part * n_tiles);
+  if (part >= (int64_t)entries * sub) return false;
+  const int s = (int)(part / entries);
+  const MTile t = g.sched[part - (int64_t)s * entries];
+  grp = t.group;
+  row0 = t.row0 + s * BM;
+  rows = min(BM, t.rows - s * BM);
+  return rows > 0;
+}
+
+// Blocks of a grid for m_tiles M tiles and n_tiles N tiles, each cut (cut_tile) or not.
+inline int64_t tile_grid(int64_t m_tiles, int64_t n_tiles, bool cut) {
+  const int64_t run = cut ? CUT_RUN : 1;
+  return 8 * run * cdiv(m_tiles * n_tiles, 8 * run);
+}
+
 // Maps blockIdx.x to (group, first row, valid rows, N tile).  Tiles are
 // enumerated M-major, N fastest; block b runs on XCD b % 8 and XCD x takes the
 // x-th contiguous eighth of the tile list.  A routed schedule of height bm (a
-// multiple of BM) is cut into bm / BM tiles an entry.  Returns false for surplus
-// blocks and for the parts of an entry past its rows.
+// multiple of BM) is cut into bm / BM tiles an entry (cut_tile).  Returns false for
+// surplus blocks and for the parts of an entry past its rows.
 template <int BM>
 __device__ __forceinline__ bool tile_for_block(const GemmDesc& g, int n_tiles, int& grp, int& row0, int& rows,
                                                int& n_tile) {
   int64_t m_total;
   int tpg = 0;
   const int sub = g.sched ? g.bm / BM : 1;
+  if (sub > 1) return cut_tile<BM>(g, sub, n_tiles, blockIdx.x >> 3, blockIdx.x & 7, grp, row0, rows, n_tile);
   if (g.sched) {
-    m_total = (int64_t)*g.sched_count * sub;
+    m_total = *g.sched_count;
   } else {
     tpg = (int)cdiv(g.dense_rows, BM);
     m_total = (int64_t)tpg * g.groups;
@@ -31,12 +69,10 @@ __device__ __forceinline__ bool tile_for_block(const GemmDesc& g, int n_tiles, i
   const int64_t m_tile = lin / n_tiles;
   n_tile = (int)(lin - m_tile * n_tiles);
   if (g.sched) {
-    const MTile t = g.sched[m_tile / sub];
-    const int s = (int)(m_tile % sub) * BM;
+    const MTile t = g.sched[m_tile];
     grp = t.group;
-    row0 = t.row0 + s;
-    rows = min(BM, t.rows - s);
-    return rows > 0;
+    row0 = t.row0;
+    rows = t.rows;
   } else {
     grp = (int)(m_tile / tpg);
     const int mt = (int)(m_tile - (int64_t)grp * tpg);
@@ -62,7 +98,7 @@ __device__ __forceinline__ bool tile_for_block_pair(const GemmDesc& gr, const Ge
   int64_t mr;
   const int sub = gr.sched ? gr.bm / BM : 1;
   if (gr.sched) {
-    mr = (int64_t)*gr.sched_count * sub;
+    mr = *gr.sched_count;
   } else {
     tpg_r = (int)cdiv(gr.dense_rows, BM);
     mr = (int64_t)tpg_r * gr.groups;
@@ -83,18 +119,17 @@ __device__ __forceinline__ bool tile_for_block_pair(const GemmDesc& gr, const Ge
     return true;
   }
   which = 0;
+  if (sub > 1) return cut_tile<BM>(gr, sub, ntr, j - per_d, (int)x, grp, row0, rows, n_tile);
   if (j - per_d >= per_r) return false;
   lin = x * per_r + (j - per_d);
   if (lin >= tr) return false;
   const int64_t m_tile = lin / ntr;
   n_tile = (int)(lin - m_tile * ntr);
   if (gr.sched) {
-    const MTile t = gr.sched[m_tile / sub];
-    const int s = (int)(m_tile % sub) * BM;
+    const MTile t = gr.sched[m_tile];
     grp = t.group;
-    row0 = t.row0 + s;
-    rows = min(BM, t.rows - s);
-    return rows > 0;
+    row0 = t.row0;
+    rows = t.rows;
   } else {
     grp = (int)(m_tile / tpg_r);
     row0 = (int)(m_tile - (int64_t)grp * tpg_r) * BM;
