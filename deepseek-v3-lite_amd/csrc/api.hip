@@ -355,19 +355,36 @@ int dsmoe_permute_noalloc(const int32_t* idx, const dsmoe_dims* dims, int32_t* o
 // both GEMMs.  Above that the 256-row tiles of the persistent kernel stay mostly
 // padding while the rows of an expert are few: a launch is a stream of weights
 // there, and what counts is how evenly its tiles fill the 256 CUs.
-// few_rows(rows, groups, n): whether the few-row kernel is the faster one for
-// `rows` routed rows over `groups` experts, n output columns (SwiGLU: 2 I).
-// Measured (us, persistent kernel against few-row kernel):
-//   E 16, D 1024, I 512, k 4 (64 tiles of 256 columns, rows per expert 25 / 50 / 83):
-//     gate/up 22 / 27 / 29 against 19 / 23 / 30, down 22 / 28 / 29 against 18 / 19 / 20;
-//   E 20, D 768, I 384, k 4 (60 tiles; 20 / 40 / 67 / 102 rows):
-//     gate/up 18 / 24 / 25 / 25 against 16 / 18 / 20 / 26, down 15 / 19 / 20 / 20 against 12 / 13 / 14 / 21.
-// With a CU's tile or more (E 64, D 2048: 704 gate/up tiles, 512 down tiles) it is the
-// slower one from 19 rows on: it reads the activations again for every 64 columns.
+// few_rows(epi, rows, groups, n, dense...): whether the few-row kernel is the faster
+// one for `rows` routed rows over `groups` experts, n output columns (SwiGLU: I), with
+// dense_groups dense problems of dense_rows rows and dense_n columns in its launch.
+// Two lines:
+//  * Weights of fewer than 256 column tiles, at most 64 rows per expert.  With a CU's
+//    tile or more (E 64, D 2048: 704 gate/up tiles, 512 down tiles) it is the slower
+//    one from 19 rows on: it reads the activations again for every 64 columns.
+//  * Its tiles of 64 rows (32 columns of h, or 64) run on the 512 places that two
+//    workgroups per CU make, in one round; a tile half counts for its weights, half
+//    for its rows.  Past that a second round starts.  Measured per GEMM (us; few-row
+//    kernel / 128-row tiles / persistent; tiles counted so):
+//    E 16, D 1024, I 512, k 4, S 1 of 1024: T 65 gate/up 19 / 23 / 24 (232), down 18 / 20
+//      / 24 (176); T 200 23 / 23 / 28 (390), 20 / 21 / 28 (326); T 256 24 / 23 / 29 (448), 20 / 21
+//      / 29 (384); T 300 (over 64 rows) 33 / 23 / 28 (524), 20 / 21 / 29.
+//    E 8, D 2048, I 1408, k 2, S 1: T 128 34 / 37 / 36 (352), 26 / 26 / 29 (256); T 200
+//      50 / 37 / 42 (539), 28 / 26 / 34 (392); one expert with every token, T 200: 51 / 43 / 42, 28 / 31 / 34.
+//    E 128, D 1024, I 128, k 1, S 1 of 1024, gate/up: T 256 21 / 23 / 29 (392), T 512 28 / 26 / 29 (528),
+//      T 1024 33 / 27 / 30 (800), T 8192 144 / 71 / 56 (4480).
+//    E 32, D 1024, I 256, k 2, S 0: T 600 16 / 23 / 23 (214), down 12 / 12 / 12 (428); T 1000
+//      23 / 23 / 24 (314), 18 / 12 / 14 (627).
 constexpr int SK_MAX_T = SK_BM;
 
-static bool few_rows(int64_t rows, int groups, int n) {
-  return cdiv(n, 256) * groups < 256 && rows <= 64 * (int64_t)groups;
+static bool few_rows(int epi, int64_t rows, int groups, int n, int64_t dense_rows, int dense_groups, int dense_n) {
+  const bool swiglu = epi == EPI_SWIGLU;
+  if (cdiv((int64_t)n * (swiglu ? 2 : 1), 256) * groups >= 256 || rows > 64 * (int64_t)groups) return false;
+  const int64_t bn = swiglu ? 32 : 64;
+  // experts with rows have a tile, and a half full one more from 64 rows on average
+  const int64_t tiles = std::max(std::min<int64_t>(rows, groups), rows / SK_BM + groups / 2);
+  const int64_t routed = (tiles + rows / SK_BM) * cdiv(n, bn) / 2;
+  return routed + cdiv(dense_rows, SK_BM) * dense_groups * cdiv(dense_n, bn) <= 512;
 }
 
 // Tiles of 128 rows (launch_small of gemm.hip) or the persistent kernel's of 256:
@@ -456,12 +473,12 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g.bm = g2.bm = bm;
   g.small_tiles = small_tiles(EPI_SWIGLU, d.T, d.E, d.I, 0, 0, 0);
   g2.small_tiles = small_tiles(EPI_STORE, d.T, d.E, d.D, 0, 0, 0);
-  if (mfr && few_rows(d.T, d.E, 2 * d.I) && gemm_sk_ok(g))
+  if (mfr && few_rows(EPI_SWIGLU, d.T, d.E, d.I, 0, 0, 0) && gemm_sk_ok(g))
     rc = launch_gemm_sk(g, EPI_SWIGLU, nullptr, st);
   else
     rc = launch_grouped_gemm(g, EPI_SWIGLU, d.dtype, nullptr, al, st);
   if (rc) return rc;
-  if (mfr && few_rows(d.T, d.E, d.D) && gemm_sk_ok(g2)) return launch_gemm_sk(g2, EPI_STORE, sorted_w, st);
+  if (mfr && few_rows(EPI_STORE, d.T, d.E, d.D, 0, 0, 0) && gemm_sk_ok(g2)) return launch_gemm_sk(g2, EPI_STORE, sorted_w, st);
   return launch_grouped_gemm(g2, EPI_STORE, d.dtype, sorted_w, al, st);
 }
 
@@ -491,6 +508,86 @@ static int launch_sk_pair(const GemmDesc& gr, const GemmDesc& gd, bool has_gd, i
   return launch_grouped_gemm(gd, epi, dtype, nullptr, gemm_mfma_eligible(gd, dtype, mf), st);
 }
 
+// The four GEMM problems of a layer forward and the kernels of the routed ones.
+struct FwdGemms {
+  GemmDesc g1, g2;    // routed: gate/up, down
+  GemmDesc s1, s2;    // shared experts (S > 0)
+  bool few1, few2;    // the few-row kernel for either GEMM
+  bool al;            // launch_grouped_gemm's allow_mfma of the routed problems
+};
+
+static FwdGemms fwd_gemms(const dsmoe_dims& d, int training, const void* x, const FwdLayout& L, bool mf) {
+  const int64_t N = (int64_t)d.T * d.k;
+  FwdGemms G;
+  GemmDesc &g1 = G.g1, &g2 = G.g2, &s1 = G.s1, &s2 = G.s2;
+  g1 = g2 = s1 = s2 = desc_zero();
+  g1.A = x; g1.lda = d.D; g1.a_rows = d.T; g1.a_map = L.sorted_token;
+  g1.B0 = L.ptrs; g1.B1 = L.ptrs + d.E; g1.ldb = d.D; g1.kseg = d.D;
+  g1.N = d.I; g1.K = d.D; g1.C = L.h; g1.ldc = d.I; g1.Gs = L.g; g1.Us = L.u;
+  // expert outputs stay in sorted order (rows written whole, in order); the
+  // combine and the backward read slot s at row slot_pos[s]
+  g2.A = L.h; g2.lda = d.I; g2.a_rows = N; g2.B0 = L.ptrs + 2 * d.E; g2.ldb = d.I; g2.kseg = d.I;
+  g2.N = d.D; g2.K = d.I; g2.C = L.o_sorted; g2.ldc = d.D;
+  const bool mfr = gemm_mfma_eligible(g1, d.dtype, mf) && gemm_mfma_eligible(g2, d.dtype, mf);
+  G.al = d.dtype == DSMOE_F32 ? mf : mfr;
+  // few rows per expert: the few-row kernel for either GEMM (never where the
+  // gate/up GEMM saves pre-activations)
+  G.few1 = G.few2 = false;
+  if (d.dtype == DSMOE_BF16 && mf && (mfr || (!training && d.T <= SK_MAX_T))) {
+    GemmDesc t1 = g1, t2 = g2;
+    t1.bm = t2.bm = SK_BM;
+    const bool ok1 = !training && gemm_sk_ok(t1), ok2 = gemm_sk_ok(t2);
+    if (d.T <= SK_MAX_T && ok1 && ok2) {
+      G.few1 = G.few2 = true;
+    } else if (mfr) {
+      G.few1 = ok1 && few_rows(EPI_SWIGLU, N, d.E, d.I, d.T, d.S, d.I_s);
+      G.few2 = ok2 && few_rows(EPI_STORE, N, d.E, d.D, d.T, d.S ? 1 : 0, d.D);
+    }
+  }
+  // the routed schedule's height follows the kernel choice
+  const int bm = G.few1 && G.few2 ? SK_BM : gemm_tile_m(mfr);
+  g1.sched = g2.sched = L.ps.sched;
+  g1.sched_count = g2.sched_count = L.ps.sched_count;
+  g1.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm);
+  g1.bm = g2.bm = bm;
+  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.T, d.S, d.I_s);
+  g2.small_tiles = small_tiles(EPI_STORE, N, d.E, d.D, d.T, d.S ? 1 : 0, d.D);
+  // gate/up: routed rows gathered from x through sorted_token, and the shared
+  // experts as S dense groups over all tokens (h_shared = [h_0 | h_1 | ...])
+  if (d.S) {
+    s1.dense_rows = d.T; s1.groups = d.S;
+    s1.A = x; s1.lda = d.D; s1.a_rows = d.T;
+    s1.B0 = L.ptrs + 3 * d.E; s1.B1 = L.ptrs + 3 * d.E + d.S; s1.ldb = d.D; s1.kseg = d.D;
+    s1.N = d.I_s; s1.K = d.D; s1.C = L.hs; s1.ldc = (int64_t)d.S * d.I_s; s1.c_group_col = d.I_s;
+    s1.Gs = L.gs; s1.Us = L.us;
+    s1.bm = gemm_tile_m(gemm_mfma_eligible(s1, d.dtype, mf));
+    // shared down projection: one GEMM with K = S * I_s summing all shared experts
+    s2.dense_rows = d.T; s2.groups = 1;
+    s2.A = L.hs; s2.lda = (int64_t)d.S * d.I_s; s2.a_rows = d.T;
+    s2.B0 = L.ptrs + 3 * d.E + 2 * d.S; s2.ldb = d.I_s; s2.kseg = d.I_s; s2.nseg = d.S;
+    s2.N = d.D; s2.K = d.S * d.I_s; s2.C = L.shared_out; s2.ldc = d.D;
+    s2.bm = gemm_tile_m(gemm_mfma_eligible(s2, d.dtype, mf));
+  }
+  return G;
+}
+
+int dsmoe_moe_fwd_kernels(const dsmoe_dims* dims, int training, int32_t* kernels) {
+  const int rc = validate(dims, true);
+  if (rc) return rc;
+  DSMOE_REQUIRE(kernels, DSMOE_ERR_INVALID, "moe_fwd_kernels: NULL output");
+  void* const aligned = reinterpret_cast<void*>(uintptr_t(256));   // never read: addresses for the alignment tests
+  const FwdLayout L = fwd_layout(*dims, training, aligned);
+  const FwdGemms G = fwd_gemms(*dims, training, aligned, L, true);
+  const auto kind = [&](const GemmDesc& g, bool few) {
+    if (few) return DSMOE_GEMM_FEW_ROWS;
+    if (!gemm_mfma_eligible(g, dims->dtype, G.al) || !gemm_qp_ok(g)) return DSMOE_GEMM_OTHER;
+    return g.small_tiles ? DSMOE_GEMM_SMALL_TILES : DSMOE_GEMM_PERSISTENT;
+  };
+  kernels[0] = kind(G.g1, G.few1);
+  kernels[1] = kind(G.g2, G.few2);
+  return DSMOE_OK;
+}
+
 int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, const void* const* w1,
                   const void* const* w2, const void* const* w3, const void* const* sw1, const void* const* sw2,
                   const void* const* sw3, const dsmoe_dims* dims, int training, void* y, int64_t* idx64,
@@ -505,7 +602,6 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   DSMOE_REQUIRE(workspace && workspace_bytes >= need, DSMOE_ERR_WORKSPACE, "moe_fwd: workspace too small");
   hipStream_t st = static_cast<hipStream_t>(stream);
   FwdLayout L = fwd_layout(d, training, workspace);
-  const int64_t N = (int64_t)d.T * d.k;
   StageTimer tm(st);
 
   // The weight pointer table goes to the device with the gate launch when it
@@ -527,36 +623,11 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   }
   const bool mf = all_aligned16(w1, d.E) && all_aligned16(w2, d.E) && all_aligned16(w3, d.E) &&
                   (d.S == 0 || (all_aligned16(sw1, d.S) && all_aligned16(sw2, d.S) && all_aligned16(sw3, d.S)));
-  // GEMM descriptors; the routed schedule height follows the kernel choice
-  GemmDesc g1 = desc_zero();
-  g1.A = x; g1.lda = d.D; g1.a_rows = d.T; g1.a_map = L.sorted_token;
-  g1.B0 = L.ptrs; g1.B1 = L.ptrs + d.E; g1.ldb = d.D; g1.kseg = d.D;
-  g1.N = d.I; g1.K = d.D; g1.C = L.h; g1.ldc = d.I; g1.Gs = L.g; g1.Us = L.u;
-  GemmDesc g2 = desc_zero();
-  g2.A = L.h; g2.lda = d.I; g2.a_rows = N; g2.B0 = L.ptrs + 2 * d.E; g2.ldb = d.I; g2.kseg = d.I;
-  // expert outputs stay in sorted order (rows written whole, in order); the
-  // combine and the backward read slot s at row slot_pos[s]
-  g2.N = d.D; g2.K = d.I; g2.C = L.o_sorted; g2.ldc = d.D;
-  const bool mfr = gemm_mfma_eligible(g1, d.dtype, mf) && gemm_mfma_eligible(g2, d.dtype, mf);
-  const bool al = d.dtype == DSMOE_F32 ? mf : mfr;
-  // few rows per expert: the few-row kernel for either GEMM (never where the
-  // gate/up GEMM saves pre-activations)
-  bool sk1 = false, sk2 = false;
-  if (d.dtype == DSMOE_BF16 && mf && (mfr || (!training && d.T <= SK_MAX_T))) {
-    GemmDesc t1 = g1, t2 = g2;
-    t1.bm = t2.bm = SK_BM;
-    const bool ok1 = !training && gemm_sk_ok(t1), ok2 = gemm_sk_ok(t2);
-    if (d.T <= SK_MAX_T && ok1 && ok2) {
-      sk1 = sk2 = true;
-    } else if (mfr) {
-      sk1 = ok1 && few_rows(N, d.E, 2 * d.I);
-      sk2 = ok2 && few_rows(N, d.E, d.D);
-    }
-  }
-  const int bm = sk1 && sk2 ? SK_BM : gemm_tile_m(mfr);
+  const FwdGemms G = fwd_gemms(d, training, x, L, mf);
+  const GemmDesc &g1 = G.g1, &g2 = G.g2, &s1 = G.s1, &s2 = G.s2;
   // (a) gate; the MFMA gate's routing launch also ranks the slots for the
   // permute (and finishes it for a call of one rank block)
-  const PermuteOut po = permute_out(L.ps, bm, L.offsets, L.sorted_slot, L.sorted_token, L.slot_pos, counts,
+  const PermuteOut po = permute_out(L.ps, g1.bm, L.offsets, L.sorted_slot, L.sorted_token, L.slot_pos, counts,
                                     training ? L.w : nullptr, L.sorted_w);
   GateOut go{logits, L.idx, idx64, L.w, weights_x, L.sel, nullptr};
   bool ranked = false;
@@ -576,43 +647,21 @@ int dsmoe_moe_fwd(const void* x, const float* gate_w, const float* gate_bias, co
   }
   tm.end();
   if (rc) return rc;
-  g1.sched = g2.sched = L.ps.sched;
-  g1.sched_count = g2.sched_count = L.ps.sched_count;
-  g1.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm);
-  g1.bm = g2.bm = bm;
-  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.T, d.S, d.I_s);
-  g2.small_tiles = small_tiles(EPI_STORE, N, d.E, d.D, d.T, d.S ? 1 : 0, d.D);
-  // (c) gate/up + SwiGLU: routed rows gathered from x through sorted_token,
-  // and the shared experts as S dense groups over all tokens (h_shared =
-  // [h_0 | h_1 | ...]), in one launch when the persistent kernel takes both
-  GemmDesc s1 = desc_zero(), s2 = desc_zero();
-  if (d.S) {
-    s1.dense_rows = d.T; s1.groups = d.S;
-    s1.A = x; s1.lda = d.D; s1.a_rows = d.T;
-    s1.B0 = L.ptrs + 3 * d.E; s1.B1 = L.ptrs + 3 * d.E + d.S; s1.ldb = d.D; s1.kseg = d.D;
-    s1.N = d.I_s; s1.K = d.D; s1.C = L.hs; s1.ldc = (int64_t)d.S * d.I_s; s1.c_group_col = d.I_s;
-    s1.Gs = L.gs; s1.Us = L.us;
-    s1.bm = gemm_tile_m(gemm_mfma_eligible(s1, d.dtype, mf));
-    // shared down projection: one GEMM with K = S * I_s summing all shared experts
-    s2.dense_rows = d.T; s2.groups = 1;
-    s2.A = L.hs; s2.lda = (int64_t)d.S * d.I_s; s2.a_rows = d.T;
-    s2.B0 = L.ptrs + 3 * d.E + 2 * d.S; s2.ldb = d.I_s; s2.kseg = d.I_s; s2.nseg = d.S;
-    s2.N = d.D; s2.K = d.S * d.I_s; s2.C = L.shared_out; s2.ldc = d.D;
-    s2.bm = gemm_tile_m(gemm_mfma_eligible(s2, d.dtype, mf));
-  }
+  // (c) gate/up + SwiGLU, routed and shared experts in one launch when the same
+  // kernel takes both
   tm.begin(ST_GEMM1);
-  rc = sk1 ? launch_sk_pair(g1, s1, d.S > 0, EPI_SWIGLU, d.dtype, mf, st)
-          : d.S ? launch_grouped_gemm_pair(g1, s1, EPI_SWIGLU, d.dtype, nullptr, al, mf, st)
-                : launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, al, st);
+  rc = G.few1 ? launch_sk_pair(g1, s1, d.S > 0, EPI_SWIGLU, d.dtype, mf, st)
+       : d.S  ? launch_grouped_gemm_pair(g1, s1, EPI_SWIGLU, d.dtype, nullptr, G.al, mf, st)
+              : launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, G.al, st);
   tm.end();
   if (rc) return rc;
   // down projections: routed rows written in expert-sorted order (row r of
   // o_sorted is sorted position r); the combine and the backward read slot s
   // at row slot_pos[s]
   tm.begin(ST_GEMM2);
-  rc = sk2 ? launch_sk_pair(g2, s2, d.S > 0, EPI_STORE, d.dtype, mf, st)
-          : d.S ? launch_grouped_gemm_pair(g2, s2, EPI_STORE, d.dtype, nullptr, al, mf, st)
-                : launch_grouped_gemm(g2, EPI_STORE, d.dtype, nullptr, al, st);
+  rc = G.few2 ? launch_sk_pair(g2, s2, d.S > 0, EPI_STORE, d.dtype, mf, st)
+       : d.S  ? launch_grouped_gemm_pair(g2, s2, EPI_STORE, d.dtype, nullptr, G.al, mf, st)
+              : launch_grouped_gemm(g2, EPI_STORE, d.dtype, nullptr, G.al, st);
   tm.end();
   if (rc) return rc;
   // (d) combine

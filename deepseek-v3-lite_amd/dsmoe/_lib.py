@@ -71,6 +71,7 @@ _SIGNATURES = {
     "dsmoe_update_bias": ([P, P, I32, F32, F32, F32, P], I32),
     "dsmoe_update_bias_f32": ([P, P, I32, F32, F32, F32, P], I32),
     "dsmoe_moe_fwd_workspace_offset": ([DIMS, I32, I32], SZ),
+    "dsmoe_moe_fwd_kernels": ([DIMS, I32, ctypes.POINTER(ctypes.c_int32)], I32),
     "dsmoe_timing_enable": ([I32], I32),
     "dsmoe_timing_read": ([ctypes.POINTER(ctypes.c_double), I32, ctypes.POINTER(ctypes.c_int)], I32),
     "dsmoe_timing_stage_name": ([I32], ctypes.c_char_p),

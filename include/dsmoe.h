@@ -238,6 +238,16 @@ int dsmoe_update_bias_f32(const float* counts, float* gate_bias, int E, float sp
 #define DSMOE_WS_SLOT_POS 6
 size_t dsmoe_moe_fwd_workspace_offset(const dsmoe_dims* dims, int training, int buffer);
 
+/* The kernels that dsmoe_moe_fwd chooses for the routed rows of a call of these
+ * dims, with 16-byte aligned tensors: kernels[0] the gate/up GEMM, kernels[1]
+ * the down projection.  For tools and tests; reads nothing on the device.  No
+ * counterpart in the reference. */
+#define DSMOE_GEMM_OTHER 0        /* fp32, or bf16 shapes that none of the following takes */
+#define DSMOE_GEMM_PERSISTENT 1   /* 256-row tiles, one workgroup per CU */
+#define DSMOE_GEMM_SMALL_TILES 2  /* 128-row tiles */
+#define DSMOE_GEMM_FEW_ROWS 3     /* 64-row tiles, weights streamed into registers */
+int dsmoe_moe_fwd_kernels(const dsmoe_dims* dims, int training, int32_t* kernels);
+
 /* ---------------------------------------------------------------------------
  * Stage timing for measurement tools (no counterpart in the reference, which
  * has no timing hooks).  While enabled, dsmoe_moe_fwd / dsmoe_moe_bwd record
