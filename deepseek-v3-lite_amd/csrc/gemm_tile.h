@@ -9,8 +9,11 @@ namespace dsmoe {
 // entry.  Parts past an entry's rows are no work, and how many there are differs
 // between entries, so the parts are listed part by part (the first of every entry,
 // the second of every entry, ...; N fastest) and the list is dealt to the XCDs in
-// runs of CUT_RUN tiles: each XCD gets an eighth of the first parts, and surplus
-// blocks come last.  Measured (us; entry by entry in eighths of the list, then so):
+// runs of CUT_RUN tiles, forth and back (0 .. 7, 7 .. 0, ...): each XCD gets an eighth of the
+// first parts, and surplus blocks come last.  An XCD's blocks go to its four shader
+// engines in turn, so a run of four loads them alike; dealt always forth, the runs of
+// every second entry (second parts where experts hold 257 to 384 rows) all fall to the same four
+// XCDs: E 16, D 1024, T 1200, down 23 us, 28 so.  Measured (us; entry by entry in eighths of the list, then so):
 //   E 8, D 2048, I 1408, k 2, T 200, one expert with every token, 64-row tiles of the
 //   down projection on a 256-row schedule: 49, 28 (one XCD held the large expert alone);
 //   E 128, D 1024, I 128, k 1, T 512, 128-row gate/up tiles: 41, 26 (surplus blocks
@@ -18,14 +21,16 @@ namespace dsmoe {
 //   E 64, D 2048, I 1408, k 6, T 1000, three experts with every token, 128-row down
 //   tiles: 181, 132; even routing 112, 111.
 // Whole parts in turn instead of runs leave XCDs idle where parts are few (E 2, D 4096,
-// I 4096, T 300: 64, 82; runs of 4: 61); runs of 1, 2 and 8 measure as runs of 4.
+// I 4096, T 300: 64, 82; runs of 4: 61); runs of 1, 2 and 8 measure as runs
+// of 4 in most shapes.
 constexpr int CUT_RUN = 4;
 
 template <int BM>
 __device__ __forceinline__ bool cut_tile(const GemmDesc& g, int sub, int n_tiles, int64_t j, int x, int& grp, int& row0,
                                          int& rows, int& n_tile) {
   const int entries = *g.sched_count;
-  const int64_t lin = (j / CUT_RUN * 8 + x) * CUT_RUN + j % CUT_RUN, part = lin / n_tiles;
+  const int64_t i = j / CUT_RUN;
+  const int64_t lin = (8 * i + (i & 1 ? 7 - x : x)) * CUT_RUN + j % CUT_RUN, part = lin / n_tiles;
   n_tile = (int)(lin - part * n_tiles);
   if (part >= (int64_t)entries * sub) return false;
   const int s = (int)(part / entries);

@@ -162,19 +162,20 @@ CUT_RUN = 4
 
 
 def tiles_cut(sched, bm: int, sub_bm: int, n_tiles: int, entries_bound: int):
-    """cut_tile: block -> (XCD, group, row0, rows, n_tile) of a schedule of height bm cut into tiles of sub_bm rows,
+    """cut_tile: block -> (XCD, index in it, group, row0, rows, n_tile) of a schedule of height bm cut into tiles of sub_bm rows,
     over the grid that tile_grid sizes from a bound on the schedule's length.  Surplus blocks are left out."""
     sub = bm // sub_bm
     out = []
     for blk in range(8 * CUT_RUN * cdiv(entries_bound * sub * n_tiles, 8 * CUT_RUN)):
         j, x = blk >> 3, blk & 7
-        part, n_tile = divmod((j // CUT_RUN * 8 + x) * CUT_RUN + j % CUT_RUN, n_tiles)
+        i = j // CUT_RUN
+        part, n_tile = divmod((8 * i + (7 - x if i % 2 else x)) * CUT_RUN + j % CUT_RUN, n_tiles)
         if part >= len(sched) * sub:
             continue
         s, entry = divmod(part, len(sched))
         grp, row0, rows = sched[entry]
         if rows > s * sub_bm:
-            out.append((x, grp, row0 + s * sub_bm, min(sub_bm, rows - s * sub_bm), n_tile))
+            out.append((x, j, grp, row0 + s * sub_bm, min(sub_bm, rows - s * sub_bm), n_tile))
     return out
 
 

@@ -241,18 +241,22 @@ def test_routed_item_order_is_a_permutation():
     ([1000] * 3 + [49] * 61, 16, 128),
     ([4] * 128, 2, 128),                       # fewer N tiles than a run
     ([150, 150], 64, 128),                     # few parts
+    ([300] * 16, 8, 128),                      # every second entry has a second part
+    ([360] * 20, 6, 128),
     ([0, 513, 0, 64, 1], 5, 64),
     ([0, 0], 4, 64),
 ], ids=str)
 def test_cut_schedules_cover_every_tile_once_and_evenly(counts, n_tiles, sub_bm):
-    """cut_tile: every tile that holds rows once, and each XCD within a run (of each contiguous stretch of such tiles)
-    of an eighth of them."""
+    """cut_tile: every tile that holds rows once; each XCD an eighth of them, and each shader engine (an XCD's blocks
+    modulo 4) a 32nd, within a run of each contiguous stretch of such tiles."""
     sched = M.routed_schedule(counts, 256)
     got = M.tiles_cut(sched, 256, sub_bm, n_tiles, sum(counts) // 256 + len(counts) + 1)
     off = np.concatenate([[0], np.cumsum(counts)])
     want = {(e, off[e] + r, min(sub_bm, c - r), n) for e, c in enumerate(counts) for r in range(0, c, sub_bm) for n in range(n_tiles)}
-    assert len(got) == len(want) and {t[1:] for t in got} == want
+    assert len(got) == len(want) and {t[2:] for t in got} == want
     share = np.bincount([t[0] for t in got], minlength=8)
     real = [rows > s * sub_bm for s in range(256 // sub_bm) for _, _, rows in sched]
     stretches = sum(a and not b for a, b in zip(real, real[1:] + [False]))
-    assert share.max() <= len(want) / 8 + M.CUT_RUN * stretches
+    assert share.max() <= len(want) / 8 + M.CUT_RUN * min(stretches, 2)
+    engines = np.bincount([4 * t[0] + t[1] % 4 for t in got], minlength=32)
+    assert engines.max() <= len(want) / 32 + min(stretches, 2)
