@@ -389,30 +389,38 @@ static bool few_rows(int epi, int64_t rows, int groups, int n, int64_t dense_row
 
 // Tiles of 128 rows (launch_small of gemm.hip) or the persistent kernel's of 256:
 // whether the small ones are faster for `rows` routed rows over `groups` experts with
-// n output columns (SwiGLU: I), and dense_groups dense problems of dense_rows rows and
-// dense_n columns in the same launch.  Two lines, by tile counts:
+// n output columns (SwiGLU: I) and k inner ones, and dense_groups dense problems of
+// dense_rows rows, dense_n columns and dense_k in the same launch.  Two lines, by tile
+// counts:
 //  * The small tiles fit the GPU at once (one for each CU with the two accumulators of
 //    the SwiGLU, else two): a launch then lasts as long as one tile, and 256-row tiles
-//    leave most CUs idle.  Measured, whole forward in a graph, persistent kernel /
-//    small gate/up / small down (us; their tile counts): E 16, D 1024, I 512, S 1: T 300
-//    79 / 74 (184) / 71 (160), T 600 81 / 80 (272) / 74 (256), T 1200 83 / 99 (440) /
-//    77 (440), T 1500 85 / 103 / 84 (528), T 2048 89 / 108 / 89 (704); operator seam of
-//    3000 even rows 63 / 57 (248) / 55 (248), 8192 rows 66 / 82 (576) / 72 (576).
+//    leave most CUs idle.  Measured, persistent kernel / small (us; the small tiles counted
+//    so), E 16, D 1024, I 512, S 1 of 1024: gate/up T 300 29 / 23 (184), T 600 29 / 28 (272), T 1200
+//    29 / 47 (440); down T 300 29 / 21 (160), T 600 29 / 23 (256), T 1200 28 / 24 (440), T 1500 28 / 25
+//    (528), T 2048 29 / 34 (704).  Operator seam, both GEMMs in a graph: 3000 even rows 49 / 43
+//    (248, 248), 8192 rows 57 / 58 (576, 576).
 //  * Store only: the 256-row tiles need a last round of CUs that is less than a quarter
-//    full (the dense tiles beside whole rounds of experts), and experts have up to 112
-//    rows, one small tile each.  E 64, D 2048, I 1408, S 2 (512 + 8 .. 40 tiles; rows per
-//    expert): T 65 (6) 268 us either way, T 200 (19) few-row kernel 290, small 271, T 333
-//    (31) 311, 280, T 450 (42) persistent 331, small 286, T 800 (75) 380, 339, T 1150
-//    (108) 376, 348, T 1300 (122) 365 both, T 1450 369, 384.  Without dense tiles (whole rounds)
-//    the persistent kernel is as fast: 400 rows 283 and few-row 285, 1200 rows 269 and 294.
-static bool small_tiles(int epi, int64_t rows, int groups, int n, int64_t dense_rows, int dense_groups, int dense_n) {
+//    full (the dense tiles beside whole rounds of experts).  Measured, persistent kernel /
+//    small (us), by rows per expert; even routing, then biases of standard deviation 0.1
+//    (a third of the experts takes most tokens):
+//    S 2, dense K twice the routed one: E 64, D 2048, I 1408, k 6: 19 rows 136 / 92, 105 / 73; 31
+//      rows 141 / 95, 111 / 92; 56 rows 142 / 100, 112 / 104; 94 rows 145 / 111, 140 / 133;
+//      E 32, D 4096, I 1408, k 4: 16 rows 125 / 93, 98 / 91; 62 rows 143 / 105, 141 / 106.  Up to 112
+//      rows (one small tile an expert).
+//    S 1, the same K: E 64, D 2048, I 1408: 16 rows 106 / 93, 77 / 69; 32 rows 113 / 96, 85 / 75;
+//      48 rows 116 / 99, 87 / 95; 104 rows 121 / 111, 113 / 129; I 512: 16 rows 51 / 42, 37 / 33;
+//      32 rows 53 / 45, 39 / 37; 48 rows 53 / 48, 40 / 46; 104 rows 55 / 54, 55 / 63; E 128, D 1024,
+//      I 512 and 1024 and E 64, I 768 and 1024 cross at the same rows.  Up to 40 rows.
+//    Without dense tiles (whole rounds) the persistent kernel is as fast.
+static bool small_tiles(int epi, int64_t rows, int groups, int n, int k, int64_t dense_rows, int dense_groups,
+                        int dense_n, int64_t dense_k) {
   const bool swiglu = epi == EPI_SWIGLU;
   const int64_t bn = swiglu ? 64 : 128;
   // an expert's last tile is half full on average
   const int64_t tiles = (rows / 128 + cdiv(groups, 2)) * cdiv(n, bn) +
                         cdiv(dense_rows, 128) * dense_groups * cdiv(dense_n, bn);
   if (tiles <= (swiglu ? 256 : 512)) return true;
-  if (swiglu || rows > 112 * (int64_t)groups) return false;
+  if (swiglu || rows > (dense_k >= 2 * (int64_t)k ? 112 : 40) * (int64_t)groups) return false;
   const int64_t big = cdiv(n, 256) * groups + cdiv(dense_rows, 256) * dense_groups * cdiv(dense_n, 256);
   return big > 256 && big < 1024 && big % 256 > 0 && big % 256 < 64;
 }
@@ -471,8 +479,8 @@ int dsmoe_grouped_swiglu_fwd(const void* x_sorted, const void* const* w1, const 
   g.sched_count = g2.sched_count = cnt;
   g.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(d.T, d.E, bm);
   g.bm = g2.bm = bm;
-  g.small_tiles = small_tiles(EPI_SWIGLU, d.T, d.E, d.I, 0, 0, 0);
-  g2.small_tiles = small_tiles(EPI_STORE, d.T, d.E, d.D, 0, 0, 0);
+  g.small_tiles = small_tiles(EPI_SWIGLU, d.T, d.E, d.I, d.D, 0, 0, 0, 0);
+  g2.small_tiles = small_tiles(EPI_STORE, d.T, d.E, d.D, d.I, 0, 0, 0, 0);
   if (mfr && few_rows(EPI_SWIGLU, d.T, d.E, d.I, 0, 0, 0) && gemm_sk_ok(g))
     rc = launch_gemm_sk(g, EPI_SWIGLU, nullptr, st);
   else
@@ -550,8 +558,8 @@ static FwdGemms fwd_gemms(const dsmoe_dims& d, int training, const void* x, cons
   g1.sched_count = g2.sched_count = L.ps.sched_count;
   g1.m_tiles_bound = g2.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm);
   g1.bm = g2.bm = bm;
-  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.T, d.S, d.I_s);
-  g2.small_tiles = small_tiles(EPI_STORE, N, d.E, d.D, d.T, d.S ? 1 : 0, d.D);
+  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.D, d.T, d.S, d.I_s, d.D);
+  g2.small_tiles = small_tiles(EPI_STORE, N, d.E, d.D, d.I, d.T, d.S ? 1 : 0, d.D, (int64_t)d.S * d.I_s);
   // gate/up: routed rows gathered from x through sorted_token, and the shared
   // experts as S dense groups over all tokens (h_shared = [h_0 | h_1 | ...])
   if (d.S) {
@@ -1069,7 +1077,7 @@ int dsmoe_grouped_swiglu_bwd(const void* x_sorted, const void* const* w1, const 
   // recompute g = X W1^T, u = X W3^T, h = silu(g) * u
   g1.B0 = B.w1; g1.B1 = B.w3; g1.C = B.h; g1.Gs = B.g; g1.Us = B.u;
   g1.sched = B.sched_f; g1.sched_count = B.cnt_f; g1.m_tiles_bound = (int32_t)sched_bound(N, d.E, bm_f); g1.bm = bm_f;
-  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, 0, 0, 0);
+  g1.small_tiles = small_tiles(EPI_SWIGLU, N, d.E, d.I, d.D, 0, 0, 0, 0);
   rc = launch_grouped_gemm(g1, EPI_SWIGLU, d.dtype, nullptr, d.dtype == DSMOE_F32 ? mf : mfr, st);
   if (rc) return rc;
   const int32_t mbound = (int32_t)sched_bound(N, d.E, BWD_BM);

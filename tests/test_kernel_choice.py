@@ -25,6 +25,9 @@ SINGLE = dict(D=1024, E=16, I=512, k=4, S=1, I_s=1024)
 @pytest.mark.parametrize("T,shape,training,want", [
     (1, WIDE, 0, (FEW, FEW)),
     (64, WIDE, 0, (FEW, FEW)),
+    (333, WIDE, 0, (PERSISTENT, SMALL)),     # a nearly empty last round of 256-row down tiles
+    (1150, WIDE, 0, (PERSISTENT, SMALL)),
+    (1300, WIDE, 0, (PERSISTENT, PERSISTENT)),
     (8192, WIDE, 0, (PERSISTENT, PERSISTENT)),
     (200, SINGLE, 0, (FEW, FEW)),
     (200, SINGLE, 1, (SMALL, FEW)),          # the few-row kernel does not save the pre-activations
@@ -49,6 +52,21 @@ def test_few_row_tiles_past_one_round():
     shape = dict(D=1024, E=32, I=256, k=2, S=0, I_s=0)
     assert _kernels(600, **shape) == (FEW, FEW)
     assert _kernels(1000, **shape) == (FEW, SMALL)
+
+
+@pytest.mark.parametrize("shape,line", [
+    (dict(D=2048, E=64, I=512, k=4, S=1, I_s=512), 40),       # shared down projection of the routed one's depth
+    (dict(D=1024, E=128, I=512, k=8, S=1, I_s=512), 40),
+    (dict(D=2048, E=64, I=1408, k=6, S=1, I_s=1408), 40),
+    (dict(D=2048, E=64, I=1408, k=6, S=1, I_s=2816), 112),    # twice as deep
+    (dict(D=1024, E=128, I=128, k=8, S=1, I_s=1024), 112),
+])
+def test_down_tiles_with_a_nearly_empty_last_round(shape, line):
+    """The rows per expert up to which 128-row tiles are taken.  (The dense tiles' share of the last round stays under a
+    quarter of the CUs here.)"""
+    T = lambda rows: rows * shape["E"] // shape["k"]
+    assert _kernels(T(line), **shape)[1] == SMALL
+    assert _kernels(T(line + 1), **shape)[1] == PERSISTENT
 
 
 def test_other_kernels_and_errors():
