@@ -402,7 +402,7 @@ static bool few_rows(int epi, int64_t rows, int groups, int n, int64_t dense_row
 //  * Store only: the 256-row tiles need a last round of CUs that is less than a quarter
 //    full (the dense tiles beside whole rounds of experts).  Measured, persistent kernel /
 //    small (us), by rows per expert; even routing, then biases of standard deviation 0.1
-//    (a third of the experts takes most tokens):
+//    (a third of the experts takes three quarters of the rows):
 //    S 2, dense K twice the routed one: E 64, D 2048, I 1408, k 6: 19 rows 136 / 92, 105 / 73; 31
 //      rows 141 / 95, 111 / 92; 56 rows 142 / 100, 112 / 104; 94 rows 145 / 111, 140 / 133;
 //      E 32, D 4096, I 1408, k 4: 16 rows 125 / 93, 98 / 91; 62 rows 143 / 105, 141 / 106.  Up to 112

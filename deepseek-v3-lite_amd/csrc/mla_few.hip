@@ -22,10 +22,10 @@
 // rounds v (relative error against float64 1.7e-3, mla.hip 2.1e-3).
 //
 // Measured at H 12, R 192, D_nope 48, D_rope 24, D_v 64 (us per call in a graph,
-// K and V built against this path): B 8, S_q 1, S_kv 1537: 74, 18 (absorb 4.0,
+// K and V built against this path): B 8, S_q 1, S_kv 1537: 54, 18 (absorb 4.0,
 // attention 9.5, sum 5.8; 5.7 MB of latent rows, 1.1 us at 5.2 TB/s: launch and
-// load latencies bound it); B 32, S_q 1, S_kv 2048: 232, 24; B 8, S_q 32: 74, 55;
-// B 1, S_q 64: 49, 36; B 1, S_q 256: 50, 55.
+// load latencies bound it); B 32, S_q 1, S_kv 600: 77, 19; B 8, S_q 16, S_kv 1537: 54, 40;
+// B 8, S_q 16, S_kv 300: 26, 28.  Where the line lies: _few in dsmoe/mla.py.
 #include <algorithm>
 #include <cstring>
 

@@ -103,15 +103,30 @@ def _prepare(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v):
     return (*(t.contiguous() for t in ts[:4]), *(w if _head_rows(w) else w.contiguous() for w in ts[4:])), bc
 
 
-def _few(S_q: int, R: int, D_nope: int, D_v: int) -> bool:
-    """Whether the attention of S_q queries runs on the latent rows
-    (csrc/mla_few.hip) instead of building K and V: where that takes fewer
-    multiplications, 3 R + D_rope for each (query, key) against
-    2 D_nope + D_rope + D_v and R (D_nope + D_v) for each key, and no more than 32
-    queries (measured at the 422m widths, S_kv 1537: 55 against 74 us at B 8 and
-    26 against 49 at B 1 with 32 queries; from 128 to 256 queries the K and V
-    path is the faster one)."""
-    return S_q <= 32 and S_q * (3 * R - 2 * D_nope - D_v) <= R * (D_nope + D_v)
+def _few(S_q: int, S_kv: int, R: int, D_nope: int, D_v: int) -> bool:
+    """Whether the attention of S_q queries of S_kv keys runs on the latent rows
+    (csrc/mla_few.hip) instead of building K and V.
+
+    Latent rows cost 3 R + D_rope for each (query, key), against 2 D_nope + D_rope +
+    D_v, and R (D_nope + D_v) for taking a query there and back, against as much for
+    each key; the latter runs on matrix cores and a query's on vector units, which
+    measures like 24 keys.  At most 32 queries.  Measured, us in a graph, latent rows /
+    K and V, at H 12, R 192, D_nope 48, D_rope 24, D_v 64 (the rule takes the former up
+    to 1, 2, 4, 10, 16, 28 queries at 33, 64, 128, 300, 600, 1537 keys):
+    1537 keys: B 1, 1 query 16 / 24, 16 queries 21 / 25, 32 26 / 25; B 8: 18 / 54, 40 / 54, 55 / 54;
+      B 2 and 4, 32 queries: 36 / 31, 40 / 38;
+    600 keys: B 4, 1 query 16 / 25, 16 queries 25 / 25; B 8, 16 queries 30 / 33;
+    300 keys: B 1, 16 queries 18 / 19; B 8, 8 queries 21 / 26, 16 28 / 26, 32 37 / 26;
+    128 keys: B 1, 1 query 16 / 14, 4 queries 17 / 14; B 8: 16 / 16, 18 / 16; B 32: 17 / 26, 24 / 26, 16
+      queries 51 / 26;
+    16 keys: 1 query, B 1 13 / 12, B 32 16 / 19; B 32, 16 queries 46 / 18.
+    At H 32, R 256, D_nope 128, D_rope 64, D_v 128: 4096 keys, B 4, 32 queries 109 / 355; 300 keys, B 8,
+    8 queries 43 / 56, 16 queries 71 / 55.  (Up to 128 keys and few batches the K and V path, one launch
+    less there, is up to 3 us faster; the latent rows keep v exact: error against float64
+    1.7e-3, with K and V 2.1e-3.)"""
+    heads = D_nope + D_v
+    pays = S_q * (24 * R * heads + S_kv * (3 * R - heads - D_nope)) <= S_kv * R * heads
+    return S_q <= 32 and (S_q == 1 or pays)
 
 
 def _head_rows(w: torch.Tensor) -> bool:
@@ -150,7 +165,7 @@ def _forward(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int, w
     """dsmoe_mla_attn_fwd (or _fwd_lse) over the batch chunks: bf16 out, the
     fp32 lse (None unless asked for) and the workspace, which holds the last
     chunk's K and V; None for a few queries, whose attention builds neither."""
-    if _few(ts[0].size(2), ts[2].size(2), ts[0].size(3), ts[5].size(1)):
+    if _few(ts[0].size(2), *ts[2].shape[1:], ts[0].size(3), ts[5].size(1)):
         return (*_forward_few(ts, bc, softmax_scale, is_causal, q_start), None)
     q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v = ts
     B, H, S_q, _ = q_nope.shape

@@ -1,5 +1,7 @@
 """GPU parity of the attention of a few queries on the latent rows (csrc/mla_few.hip) against the float64 oracle,
 with the bar of tests/test_gpu_mla.py, at the edges of its tiles, key ranges and load forms."""
+from unittest import mock
+
 import numpy as np
 import pytest
 import torch
@@ -11,11 +13,26 @@ pytestmark = pytest.mark.gpu
 
 
 def _run(ts, sc, causal, q_start):
+    """The call on the latent rows, also where the rule prefers K and V."""
     import dsmoe.mla as M
-    assert M._few(ts[0].size(2), ts[2].size(2), ts[0].size(3), ts[5].size(1)), "not the path under test"
-    out = M.mla_attention(*ts, sc, is_causal=causal, q_start=q_start)
+    with mock.patch.object(M, "_few", lambda *a: True):
+        out = M.mla_attention(*ts, sc, is_causal=causal, q_start=q_start)
     torch.cuda.synchronize()
     return out
+
+
+def test_the_rule_chooses_the_path():
+    """mla_attention takes the path that _few names: the C function it calls."""
+    import dsmoe._lib as L
+    import dsmoe.mla as M
+    for S_q, S_kv in ((1, 16), (4, 16), (10, 300), (12, 300), (33, 4096)):
+        ts, sc = _inputs(1, 2, S_q, S_kv, 192, 48, 24, 64, seed=S_q)
+        lib = mock.Mock(wraps=L.load())
+        with mock.patch.object(L, "load", lambda: lib):
+            M.mla_attention(*ts, sc, is_causal=False, q_start=0)
+        assert lib.dsmoe_mla_attn_few.called == M._few(S_q, S_kv, 192, 48, 64)
+        assert lib.dsmoe_mla_attn_few.called != lib.dsmoe_mla_attn_fwd_heads.called
+    torch.cuda.synchronize()
 
 
 def _check(out, ts, sc, causal, q_start):
@@ -92,7 +109,7 @@ def test_key_ranges(B, H, S_q, S_kv, R, Dn, Dr, Dv, causal, q_start):
     import dsmoe._lib as L
     import dsmoe.mla as M
     ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=S_q)
-    assert not M._few(S_q, R, Dn, Dv)
+    assert not M._few(S_q, S_kv, R, Dn, Dv)
     w = torch.cat([ts[4], ts[5]], 1)
     ins, bc = M._prepare(*ts[:4], w[:, :Dn], w[:, Dn:])
     out, lse, ws = M._forward(ins, bc, sc, causal, q_start, want_lse=True)

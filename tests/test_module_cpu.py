@@ -312,3 +312,10 @@ def test_mla_operator_rejects_host_tensors_and_bad_dims():
                       torch.zeros(1, 8, 8, dtype=torch.bfloat16), torch.zeros(1, 8, 8, dtype=torch.bfloat16), 0.3)
     with pytest.raises(ValueError, match="256"):
         _check_mla_dim_limits(300, 8, 8, 8)
+
+
+@pytest.mark.parametrize("S_kv,most", [(16, 1), (33, 1), (64, 2), (128, 4), (300, 10), (600, 16), (1537, 28), (4096, 32)])
+def test_attention_takes_the_latent_rows_up_to(S_kv, most):
+    """dsmoe.mla._few at the 422m widths: queries over S_kv keys on the latent rows, more than `most` on K and V."""
+    from dsmoe.mla import _few
+    assert [q for q in range(1, 65) if _few(q, S_kv, 192, 48, 64)] == list(range(1, most + 1))
