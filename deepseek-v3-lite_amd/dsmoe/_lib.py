@@ -8,6 +8,7 @@ unsupported shapes raise ValueError, HIP errors raise RuntimeError.
 from __future__ import annotations
 
 import ctypes
+import warnings
 from pathlib import Path
 from typing import Iterable, Sequence
 
@@ -92,21 +93,26 @@ _layer_fns = None
 
 def layer_fns():
     """(host module, dsmoe_moe_fwd, dsmoe_moe_bwd_ex) of the eager layer path: the
-    two functions take their host pointer arrays as bytes (the host module's)."""
+    two functions take their host pointer arrays as bytes (the host module's).  None,
+    with a warning the first time, when the host module is not built or was built
+    for another torch: the layer's torch.library operators then serve every call."""
     global _layer_fns
     if _layer_fns is None:
         lib = load()
         try:
             from . import _host
         except ImportError as e:
-            raise ImportError(f"dsmoe: {LIB_PATH.parent / '_host.so'} is not built or does not load ({e}); run "
-                              "__graft_entry__.build() (or `python -m dsmoe.build` in deepseek-v3-lite_amd/)") from e
+            _layer_fns = ()
+            warnings.warn(f"dsmoe: {LIB_PATH.parent / '_host.so'} is not built or does not load ({e}); eager layer calls "
+                          "take up to 1 ms of host time more through torch.library operators.  Run "
+                          "__graft_entry__.build() (or `python -m dsmoe.build` in deepseek-v3-lite_amd/)", RuntimeWarning)
+            return None
         fns = []
         for name in ("dsmoe_moe_fwd", "dsmoe_moe_bwd_ex"):
             args, res = _SIGNATURES[name]
             fns.append(ctypes.CFUNCTYPE(res, *[P if a is PP else a for a in args])((name, lib)))
         _layer_fns = (_host, *fns)
-    return _layer_fns
+    return _layer_fns or None
 
 
 def load() -> ctypes.CDLL:

@@ -358,9 +358,10 @@ class _LayerFn(torch.autograd.Function):
 def _eager_layer(x, gate_w, gate_bias, weights, masters, E, S, k, route_scale, training):
     """The layer of a plain eager call: (y, idx64, weights_x, counts), or None
     when the call is not one (the operator path then checks and runs it)."""
-    if not _plain_eager():
+    fns = L.layer_fns() if _plain_eager() else None
+    if fns is None:
         return None
-    found = L.layer_fns()[0].scan(weights, masters, x, gate_w, gate_bias, E, S, k)
+    found = fns[0].scan(weights, masters, x, gate_w, gate_bias, E, S, k)
     if found is None:
         return None
     I, I_s, needs_grad, arrays = found

@@ -163,3 +163,18 @@ def test_module_reads_replaced_and_computed_weights():
         P.remove_parametrizations(m.experts[0].w3, "weight")
         d = m(x)
     assert torch.equal(c, d) and not torch.equal(b, c)
+
+
+def test_without_the_host_module(monkeypatch):
+    """The layer without dsmoe/_host.so: the same results through the operators."""
+    import sys
+
+    import dsmoe._lib as L
+    args = _args()
+    want = _step(*args, False)
+    monkeypatch.setattr(L, "_layer_fns", None)
+    monkeypatch.setitem(sys.modules, "dsmoe._host", None)
+    monkeypatch.delattr("dsmoe._host", raising=False)
+    with pytest.warns(RuntimeWarning, match="_host.so"):
+        got = _step(*args, False)
+    assert all(map(_same, want[0], got[0])) and all(map(_same, want[1], got[1]))

@@ -2,6 +2,8 @@
 constructor contract, state_dict keys, buffers, error on CPU forward, balance
 metric and bias update from planted routings, config-compat helper.  Mirrors
 the reference's tests/test_models.py:287-389,757-800 and tests/test_force_back.py."""
+import sys
+
 import pytest
 import torch
 
@@ -319,3 +321,16 @@ def test_attention_takes_the_latent_rows_up_to(S_kv, most):
     """dsmoe.mla._few at the 422m widths: queries over S_kv keys on the latent rows, more than `most` on K and V."""
     from dsmoe.mla import _few
     assert [q for q in range(1, 65) if _few(q, S_kv, 192, 48, 64)] == list(range(1, most + 1))
+
+
+def test_without_the_host_module_the_operators_serve_layer_calls(monkeypatch, recwarn):
+    """dsmoe/_host.so missing or built for another torch: a warning, once, and the eager path steps aside."""
+    import dsmoe._lib as L
+    from dsmoe import ops
+    monkeypatch.setattr(L, "_layer_fns", None)
+    monkeypatch.setitem(sys.modules, "dsmoe._host", None)      # the import then raises ImportError
+    monkeypatch.delattr("dsmoe._host", raising=False)
+    t = torch.zeros(1)
+    for _ in range(2):
+        assert ops._eager_layer(t, t, t, [], [], 1, 0, 1, 1.0, None) is None
+    assert [w.category for w in recwarn if "_host.so" in str(w.message)] == [RuntimeWarning]
