@@ -171,6 +171,15 @@ def stack_array(t: torch.Tensor):
     return ctypes.cast(arr, PP), arr  # keep `arr` alive while the call runs
 
 
+def restored(ts: Sequence[torch.Tensor]) -> list:
+    """Saved tensors of a backward as the kernels read them, contiguous: a saved-tensor
+    hook may hand back equal tensors of other strides.  On another device than the
+    first they are not equal ones: RuntimeError."""
+    if any(t.device != ts[0].device for t in ts):
+        raise RuntimeError("dsmoe: saved tensors came back on different devices")
+    return [t.contiguous() for t in ts]
+
+
 def stream_ptr(device: torch.device):
     """hipStream_t of the device's current stream."""
     index = device.index if device.index is not None else torch.cuda.current_device()

@@ -291,7 +291,7 @@ class _MlaAttentionFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        *ts, out, lse = ctx.saved_tensors
+        *ts, out, lse = L.restored(ctx.saved_tensors)
         bc, softmax_scale, is_causal, q_start = ctx.args
         with torch.autocast(dout.device.type, enabled=False):
             dq_nope, dq_pe, dkv, dk_pe = mla_attention_bwd_heads(ts, bc, out, lse, dout, softmax_scale, is_causal,

@@ -269,7 +269,8 @@ def _moe_fwd_backward(ctx, dy, _didx, _dwx, _dcounts, _dws):
         return (None, None, None, [None] * len(weights), [None] * n_masters) + rest
     if not training:
         raise RuntimeError("dsmoe: forward ran without saving activations for backward")
-    g = moe_bwd_op(x, gate_w, list(weights), _c(dy), ws, E, S, k, I, I_s, rs, n_masters > 0)
+    x, gate_w, ws, *weights = L.restored((x, gate_w, ws, *weights))
+    g = moe_bwd_op(x, gate_w, weights, _c(dy), ws, E, S, k, I, I_s, rs, n_masters > 0)
     if n_masters:
         return (g[0], g[1], None, [None] * len(weights), list(g[2:])) + rest
     return (g[0], g[1], None, list(g[2:]), []) + rest
@@ -333,10 +334,11 @@ class _LayerFn(torch.autograd.Function):
             raise RuntimeError("dsmoe: forward ran without saving activations for backward")
         dy = _c(dy)
         host, _, bwd = L.layer_fns()
-        # a saved-tensor hook may hand back tensors of another kind or place than it
-        # was given; those go through the operator, as do the observers' calls
+        # a saved-tensor hook may hand back tensors of other strides than it was given;
+        # those go through the operator, as do the observers' calls
         found = host.scan(weights, [], x, gate_w, None, E, S, k) if _plain_eager() else None
         if found is None or found[:2] != (I, I_s) or ws.device != x.device or not ws.is_contiguous():
+            x, gate_w, ws, *weights = L.restored((x, gate_w, ws, *weights))
             g = moe_bwd_op(x, gate_w, weights, dy, ws, E, S, k, I, I_s, rs, masters)
             dx, dgw, dws = g[0], g[1], g[2:]
         else:
@@ -487,7 +489,7 @@ class _GroupedSwiGLUFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
-        x_sorted, w1, w2, w3, off = ctx.saved_tensors
+        x_sorted, w1, w2, w3, off = L.restored(ctx.saved_tensors)
         dev = x_sorted.device
         N, D = x_sorted.shape
         E, I, _ = w1.shape

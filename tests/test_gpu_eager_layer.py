@@ -96,7 +96,6 @@ def test_saved_tensor_hooks_and_backward_under_a_mode():
     with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.clone(), lambda t: t.clone()):
         got = _step(x, gw, gb, ws, dy, False)[1]
     assert len(packed) == 3 + sum(map(len, ws)) and all(map(_same, want, got))
-    # weights that come back with other strides go through the operator, which makes no difference to the values
     with torch.autograd.graph.save_on_cpu():
         got = _step(x, gw, gb, ws, dy, False)[1]
     assert all(map(_same, want, got))
@@ -108,6 +107,41 @@ def test_saved_tensor_hooks_and_backward_under_a_mode():
         y.backward(dy)
     assert any("dsmoe.moe_bwd" in n for n in seen.names)
     assert all(map(_same, want, [t.grad for t in (x, gw, *[t for ts in ws for t in ts])]))
+
+
+def _other_strides(t):
+    """An equal tensor, its elements two apart."""
+    return torch.stack([t, t], -1)[..., 0]
+
+
+@pytest.mark.parametrize("path", ["eager", "operator", "seam", "attention"])
+def test_saved_tensors_that_come_back_with_other_strides(path):
+    """A saved-tensor hook may hand back equal tensors of other strides: the same gradients.  Tensors on another device
+    are an error, before any kernel."""
+    from dsmoe import grouped_moe_dispatch
+    from dsmoe.mla import mla_attention
+    from tests.test_gpu_mla import _inputs
+    hooks = torch.autograd.graph.saved_tensors_hooks
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16().requires_grad_()
+    if path in ("eager", "operator"):
+        args = _args()
+        run = lambda: _step(*args, path == "operator")[1]
+    elif path == "seam":
+        ins = (n(40, 64), n(3, 32, 64), n(3, 64, 32), n(3, 32, 64), n(40))
+        off = torch.tensor([0, 7, 7, 40], device=DEV)
+        run = lambda: torch.autograd.grad(grouped_moe_dispatch(*ins, off).float().square().sum(), ins)
+    else:
+        ins, sc = _inputs(2, 3, 70, 70, 64, 32, 16, 24, seed=1)
+        ins = [t.requires_grad_() for t in ins]
+        run = lambda: torch.autograd.grad(mla_attention(*ins, sc, is_causal=True).float().square().sum(), ins)
+    want = run()
+    with hooks(lambda t: t, _other_strides):
+        got = run()
+    assert all(map(_same, want, got))
+    with hooks(lambda t: t, lambda t: t.cpu() if t.dim() > 1 and t.dtype == torch.bfloat16 else t):
+        with pytest.raises(RuntimeError, match="device"):
+            run()
 
 
 def test_no_gradient_of_gradients():
