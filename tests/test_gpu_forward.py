@@ -464,16 +464,11 @@ def test_update_bias_with_fractional_counts():
     assert not torch.equal(gate.bias.cpu(), truncated)             # integer truncation would differ
 
 
-@pytest.mark.parametrize("training", [False, True])
-@pytest.mark.parametrize("case,skew", [
-    (CS.Case("few_unfilled", 65, 256, 16, 128, 2, 1, 128, torch.bfloat16, "normal"), False),   # both GEMMs few-row
-    (CS.Case("few_unfilled", 190, 256, 4, 256, 1, 1, 128, torch.bfloat16), True),   # one expert with every row: 64-row parts
-    (CS.Case("few_unfilled", 256, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False),  # at the line: 64 rows each
-    (CS.Case("few_down", 70, 2048, 64, 256, 4, 2, 256, torch.bfloat16, "normal"), False),   # gate/up alone, down on 128-row tiles
-], ids=lambda c: str(c) if isinstance(c, bool) else f"{c.name}_T{c.T}")
-def test_few_rows_per_expert(case, skew, training):
-    """More than 64 tokens with few rows per expert: the few-row GEMM on schedules of its own height and of 256 rows,
-    beside the other kernels."""
+def _check_choice(case, skew, training, want):
+    """The layer against the oracle; want: the kernels of gate/up and down, by initial (few-row, small tiles, persistent)."""
+    from tests.test_kernel_choice import FEW, PERSISTENT, SMALL, _kernels
+    kinds = {"F": FEW, "S": SMALL, "P": PERSISTENT}
+    assert _kernels(case.T, case.D, case.E, case.I, case.k, case.S, case.I_s, int(training)) == tuple(kinds[w] for w in want)
     x, p, _ = CS.make_inputs(case)
     if skew:
         p = R.MoEParams(p.gate_w, torch.tensor([0.0, 5.0, 0.0, 0.0]), p.w1, p.w2, p.w3, p.sw1, p.sw2, p.sw3)
@@ -489,16 +484,36 @@ def test_few_rows_per_expert(case, skew, training):
     torch.testing.assert_close(y.cpu().float(), ref.float(), rtol=2e-2, atol=2e-2)
 
 
+def _choice_id(v):
+    return f"{v.name}_T{v.T}" if isinstance(v, CS.Case) else str(v)
+
+
 @pytest.mark.parametrize("training", [False, True])
-@pytest.mark.parametrize("case,skew", [
-    (CS.Case("small_both", 300, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False),   # about 75 rows each
-    (CS.Case("small_edges", 200, 320, 2, 192, 2, 2, 64, torch.bfloat16), False),   # partial N tile, 200 = 128 + 72 rows
-    (CS.Case("small_skew", 390, 256, 4, 128, 1, 1, 192, torch.bfloat16), True),    # one expert with every row: 3 x 128 + 6
-    (CS.Case("small_alone", 513, 256, 8, 128, 3, 0, 0, torch.bfloat16, "normal"), False),   # no shared expert
-    (CS.Case("small_tail", 130, 2048, 64, 128, 4, 1, 128, torch.bfloat16, "normal"), False),   # down: 512 + 8 big tiles
-    (CS.Case("past_small", 2050, 1088, 12, 320, 4, 2, 192, torch.bfloat16, "normal"), False),  # the persistent kernel
-], ids=lambda c: str(c) if isinstance(c, bool) else f"{c.name}_T{c.T}")
-def test_small_tiles(case, skew, training):
+@pytest.mark.parametrize("case,skew,want,want_training", [
+    (CS.Case("few_unfilled", 65, 256, 16, 128, 2, 1, 128, torch.bfloat16, "normal"), False, "FF", "SF"),
+    (CS.Case("few_unfilled", 190, 256, 4, 256, 1, 1, 128, torch.bfloat16), True, "FF", "SF"),  # one expert with every row: 64-row parts
+    (CS.Case("few_unfilled", 256, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False, "FF", "SF"),  # at the line: 64 rows each
+    (CS.Case("few_gate_up", 70, 2048, 64, 256, 4, 2, 256, torch.bfloat16, "normal"), False, "FS", "SS"),
+    (CS.Case("few_down", 200, 512, 16, 1024, 4, 2, 1024, torch.bfloat16, "normal"), False, "PF", "PF"),
+    (CS.Case("few_gate_up", 500, 1024, 64, 128, 8, 1, 128, torch.bfloat16, "normal"), False, "FP", "SP"),
+], ids=_choice_id)
+def test_few_rows_per_expert(case, skew, want, want_training, training):
+    """More than 64 tokens with few rows per expert: the few-row GEMM on schedules of its own height and of 256 rows,
+    beside the other kernels."""
+    _check_choice(case, skew, training, want_training if training else want)
+
+
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("case,skew,want,want_training", [
+    (CS.Case("small_both", 300, 1024, 16, 512, 4, 1, 1024, torch.bfloat16, "normal"), False, "SS", "SS"),   # about 75 rows each
+    (CS.Case("small_edges", 200, 320, 2, 192, 2, 2, 64, torch.bfloat16), False, "SS", "SS"),   # partial N tile, 200 = 128 + 72 rows
+    (CS.Case("small_skew", 390, 256, 4, 128, 1, 1, 192, torch.bfloat16), True, "SS", "SS"),    # one expert with every row: 3 x 128 + 6
+    (CS.Case("small_alone", 513, 256, 8, 128, 3, 0, 0, torch.bfloat16, "normal"), False, "SS", "SS"),   # no shared expert
+    (CS.Case("small_tail", 130, 2048, 64, 128, 4, 1, 128, torch.bfloat16, "normal"), False, "FS", "SS"),   # down: 512 + 8 big tiles
+    (CS.Case("small_gate_up", 1000, 1024, 8, 128, 8, 1, 128, torch.bfloat16), False, "SP", "SP"),
+    (CS.Case("past_small", 2050, 1088, 12, 320, 4, 2, 192, torch.bfloat16, "normal"), False, "PP", "PP"),  # partial 256-row tiles
+], ids=_choice_id)
+def test_small_tiles(case, skew, want, want_training, training):
     """Launches of few tiles on 128-row tiles, routed and shared experts in one launch; past the line the persistent
-    kernel with partial tiles."""
-    test_few_rows_per_expert(case, skew, training)
+    kernel."""
+    _check_choice(case, skew, training, want_training if training else want)

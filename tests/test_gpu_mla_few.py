@@ -147,3 +147,26 @@ def test_gradients():
     o.transpose(1, 2).backward(dout.double())
     for a, b in zip((*ins, w), (qn, qp, kv, pe, w64)):
         assert (a.grad.double() - b.grad).abs().max() <= 2e-2 + 2e-2 * b.grad.abs().max()
+
+
+@pytest.mark.parametrize("B,bc,H,S_q,S_kv,few,grows", [
+    (3, 2, 4, 1, 90, True, False),
+    (7, 4, 32, 16, 1024, True, True),         # the last chunk takes more key ranges and a larger workspace
+    (3, 2, 5, 70, 300, False, False),
+    (3, 2, 16, 512, 1024, False, True),       # the first chunk takes one range, the last several
+])
+def test_uneven_batch_chunks(monkeypatch, B, bc, H, S_q, S_kv, few, grows):
+    """Calls beyond one launch's rows: batch chunks, the last one shorter."""
+    import dsmoe._lib as L
+    import dsmoe.mla as M
+    ts, sc = _inputs(B, H, S_q, S_kv, 16, 16, 8, 16, seed=B)
+    monkeypatch.setattr(M, "_few", lambda *a: few)
+    monkeypatch.setattr(M, "_ROWS_PER_CALL", bc * H * (-(-S_kv // 64) * 64) + 1)
+    assert M._prepare(*ts)[1] == bc
+    size = L.load().dsmoe_mla_attn_few_workspace_size if few else L.load().dsmoe_mla_attn_workspace_size
+    sizes = []
+    for n in (bc, B % bc):
+        d = M._dims(ts[0][:n], ts[1][:n], ts[2][:n], ts[5], sc, True, S_kv - S_q)
+        sizes.append(int(size(d)))
+    assert (sizes[1] > sizes[0]) == grows
+    _check(M.mla_attention(*ts, sc, is_causal=True, q_start=S_kv - S_q), ts, sc, True, S_kv - S_q)
