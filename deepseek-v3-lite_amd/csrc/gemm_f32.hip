@@ -4,7 +4,9 @@
 // models/moe.py:127-131,166-179; backward (XGemm): dh, dx and the weight
 // gradients, operand layouts as listed in gemm_x.hip.  Every product is an
 // fp32 product accumulated in fp32 (v_mfma_f32_32x32x2_f32), the K range in
-// ascending slabs by one workgroup per output tile: no atomics, no split.
+// ascending slabs by one workgroup per output tile, no atomics.  The shared experts'
+// weight gradients, whose K is all tokens, are cut along K into 1 to 8 parts by shape
+// (xgemm_f32_ksplit); wgrad_reduce_kernel adds the parts in ascending order.
 //
 // What bounds it: the fp32 matrix rate, 64 cycles per 32x32x2 MFMA and SIMD
 // (157 TFLOP/s; the vector FMA units without packed instructions reach half of
@@ -452,11 +454,6 @@ static bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) =
 template <auto Kern, class... Args>
 static int f_launch(int64_t grid, size_t lds, hipStream_t st, const char* what, const Args&... args) {
   if (grid <= 0) return DSMOE_OK;
-  if (lds > 64 * 1024) {
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void*)Kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (attr != hipSuccess) return fail(DSMOE_ERR_HIP, std::string(what) + ": cannot raise LDS limit");
-  }
   hipLaunchKernelGGL(Kern, dim3((unsigned)grid), dim3(256), lds, st, args...);
   return check_launch(what);
 }
@@ -480,6 +477,7 @@ int launch_gemm_f32(const GemmDesc& gr, const GemmDesc* gd, int epi, const float
   const bool vec = tables_aligned && f_vec(gr) && (!gd || f_vec(*gd));
   const int64_t grid = 8 * (f_share(gr) + (gd ? f_share(*gd) : 0));
   constexpr size_t tile = sizeof(float) * FTile<F_FK_ROWS, false>::FLOATS;
+  static_assert(3 * tile <= 64 * 1024, "default LDS limit");
   const GemmDesc& d = gd ? *gd : gr;
   const int has = gd ? 1 : 0;
   if (epi == EPI_SWIGLU)
@@ -504,6 +502,7 @@ static int f_bwd(const XGemm& g, bool vec, hipStream_t st) {
   constexpr bool AK = EPI == XE_WGRAD;
   constexpr int FK = AK ? F_FK_WGRAD : F_FK_ROWS;
   constexpr size_t lds = sizeof(float) * (FTile<FK, AK>::FLOATS + FTile<FK, true>::FLOATS);
+  static_assert(lds <= 64 * 1024, "default LDS limit");
   int64_t m;
   if (g.sched_mode == XS_ROUTED)
     m = (int64_t)g.m_tiles_bound * (g.bm / FB);
