@@ -274,7 +274,7 @@ def _project_kv_grads(ctx_kv, wkv_b_k, wkv_b_v, dkv, dk_pe):
 class _MlaAttentionFunction(torch.autograd.Function):
 
     @staticmethod
-    def forward(ctx, q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, softmax_scale, is_causal, q_start):
+    def forward(ctx, q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, softmax_scale, is_causal, q_start, grad):
         global hip_calls
         out_dtype = q_nope.dtype
         ctx.dtypes = tuple(t.dtype for t in (q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v))
@@ -283,7 +283,11 @@ class _MlaAttentionFunction(torch.autograd.Function):
         hip_calls += 1
         # the backward runs on the bf16 operands the kernels saw, and on the
         # forward's K and V when one launch covered the batch (B H pad64(S_kv)
-        # (DQKp + DVp) bf16, held until the backward); otherwise it rebuilds them
+        # (DQKp + DVp) bf16, held until the backward); otherwise it rebuilds them.
+        # Head views of a weight are saved as copies (the backward's kernels take
+        # contiguous ones): the weight may be written in place before the backward
+        if grad:
+            ts = tuple(t.contiguous() for t in ts)
         ctx.save_for_backward(*ts, out, lse)
         ctx.kv_ws = kv_ws if bc >= ts[0].size(0) else None   # (None too after a few queries)
         ctx.args = (bc, softmax_scale, is_causal, q_start)
@@ -299,7 +303,7 @@ class _MlaAttentionFunction(torch.autograd.Function):
             ctx.kv_ws = None
             dctx_kv, dctx_pe, dwk, dwv = _project_kv_grads(ts[2], ts[4], ts[5], dkv, dk_pe)
         grads = (dq_nope, dq_pe, dctx_kv, dctx_pe, dwk, dwv)
-        return tuple(g.to(dt) for g, dt in zip(grads, ctx.dtypes)) + (None, None, None)
+        return tuple(g.to(dt) for g, dt in zip(grads, ctx.dtypes)) + (None,) * 4
 
 
 def mla_attention(q_nope: torch.Tensor, q_pe: torch.Tensor, ctx_kv: torch.Tensor, ctx_pe: torch.Tensor,
@@ -309,8 +313,9 @@ def mla_attention(q_nope: torch.Tensor, q_pe: torch.Tensor, ctx_kv: torch.Tensor
 
     ``q_start`` offsets the query positions in the KV context so a cached
     mid-sequence prefill stays causal."""
-    return _MlaAttentionFunction.apply(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v, softmax_scale, is_causal,
-                                       q_start)
+    ts = (q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v)
+    grad = torch.is_grad_enabled() and any(t.requires_grad for t in ts)
+    return _MlaAttentionFunction.apply(*ts, softmax_scale, is_causal, q_start, grad)
 
 
 triton_mla_attention = mla_attention

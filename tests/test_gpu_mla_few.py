@@ -170,3 +170,22 @@ def test_uneven_batch_chunks(monkeypatch, B, bc, H, S_q, S_kv, few, grows):
         sizes.append(int(size(d)))
     assert (sizes[1] > sizes[0]) == grows
     _check(M.mla_attention(*ts, sc, is_causal=True, q_start=S_kv - S_q), ts, sc, True, S_kv - S_q)
+
+
+@pytest.mark.parametrize("S_q", [3, 70])
+def test_weights_written_between_forward_and_backward(S_q):
+    """The per-head views of one weight that is written in place after the forward (an optimizer step of another graph):
+    the gradients of the forward that ran."""
+    from dsmoe.mla import mla_attention
+    ts, sc = _inputs(2, 3, S_q, 300, 64, 32, 16, 24, seed=7, wscale=0.3)
+    w = torch.cat([ts[4], ts[5]], 1).requires_grad_()
+    ins = [t.clone().requires_grad_() for t in ts[:4]]
+    dout = torch.randn(2, S_q, 3, 24, device=DEV).bfloat16()
+    grads = []
+    for write in (False, True):
+        out = mla_attention(*ins, w[:, :32], w[:, 32:], sc, is_causal=True, q_start=300 - S_q)
+        if write:
+            with torch.no_grad():
+                w.zero_()
+        grads.append(torch.autograd.grad(out, [*ins, w], dout))
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
