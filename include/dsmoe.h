@@ -275,13 +275,18 @@ const char* dsmoe_timing_stage_name(int stage);
  * and D_nope + D_rope <= 256 (DSMOE_ERR_UNSUPPORTED).  The workspace holds the
  * materialised K and V of every (batch, head), B * H * pad64(S_kv) *
  * (DQKp + DVp) * 2 bytes, and for calls of few query blocks the partial results
- * of their key ranges (at most 512 blocks of 128 queries, fp32): DQKp = 2 D_nope + D_rope (D_nope + D_rope when
- * that exceeds 256) and DVp = D_v, each rounded up to a multiple of 16 and 32
- * (dsmoe_mla_attn_workspace_size gives the figure; about 2.7 GB at B 1,
+ * of their key ranges (at most 512 blocks of 128 queries, fp32): DQKp = 2 D_nope +
+ * D_rope (D_nope + D_rope when that exceeds 256) and DVp = D_v, each rounded up to a
+ * multiple of 16 and 32 (dsmoe_mla_attn_workspace_size gives the figure; about 2.7 GB at B 1,
  * H 128, S_kv 32768, D_nope 128, D_rope 64, D_v 128).  Row indices are 32-bit:
  * a call needs B * H * pad64(S_kv) and B * H * S_q below 2^22
  * (DSMOE_ERR_UNSUPPORTED otherwise); dsmoe.mla splits larger calls by batch,
- * so one batch's H * S_kv and H * S_q must stay below 2^22. */
+ * so one batch's H * S_kv and H * S_q must stay below 2^22.
+ * A workspace without room for the key ranges (K and V plus 256 bytes, as sized
+ * for a call that needs none) is accepted: the call then runs on one range, which
+ * rounds the probabilities against another running maximum and sums in another
+ * order, so the same call gives slightly different bits with the two sizes.  With
+ * dsmoe_mla_attn_workspace_size bytes the ranges depend on dims alone. */
 typedef struct dsmoe_mla_dims {
   int32_t B, H, S_q, S_kv;
   int32_t R;          /* kv_lora_rank        */
@@ -328,7 +333,7 @@ int dsmoe_mla_attn_few(const void* q_nope, const void* q_pe, const void* ctx_kv,
                        const dsmoe_mla_dims* dims, void* out, float* lse, void* workspace, size_t workspace_bytes,
                        void* stream);
 /* K and V of every (batch, head) into kv_ws (dsmoe_mla_attn_workspace_size
- * bytes), the first launch of dsmoe_mla_attn_fwd on its own: for a backward
+ * bytes, or K and V plus 256), the first launch of dsmoe_mla_attn_fwd on its own: for a backward
  * whose caller did not keep the forward's workspace.  No counterpart in the
  * reference (its backward recomputes everything, models/mla_triton.py:269-296). */
 int dsmoe_mla_attn_kv(const void* ctx_kv, const void* ctx_pe, const void* wkv_b_k, const void* wkv_b_v,
