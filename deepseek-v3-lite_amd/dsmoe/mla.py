@@ -103,30 +103,31 @@ def _prepare(q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v):
     return (*(t.contiguous() for t in ts[:4]), *(w if _head_rows(w) else w.contiguous() for w in ts[4:])), bc
 
 
-def _few(S_q: int, S_kv: int, R: int, D_nope: int, D_v: int) -> bool:
+def _few(B: int, H: int, S_q: int, S_kv: int, R: int, D_nope: int, D_v: int) -> bool:
     """Whether the attention of S_q queries of S_kv keys runs on the latent rows
-    (csrc/mla_few.hip) instead of building K and V.
+    (csrc/mla_few.hip) instead of building K and V; B batches in a launch, at most 32
+    queries.
 
     Latent rows cost 3 R + D_rope for each (query, key), against 2 D_nope + D_rope +
     D_v, and R (D_nope + D_v) for taking a query there and back, against as much for
     each key; the latter runs on matrix cores and a query's on vector units, which
-    measures like 24 keys.  At most 32 queries.  Measured, us in a graph, latent rows /
-    K and V, at H 12, R 192, D_nope 48, D_rope 24, D_v 64 (the rule takes the former up
-    to 1, 2, 4, 10, 16, 28 queries at 33, 64, 128, 300, 600, 1537 keys):
+    measures like 24 keys.  Up to 768 (query, head) rows in all that way hides behind
+    the launches' latency; there the latent rows are taken whatever the keys, also
+    over caches of up to 200 keys, where K and V are up to 5 us faster: v stays exact
+    (error against float64 2.0e-3 over short caches, with K and V 2.7e-3).  Measured, us
+    in a graph, latent rows / K and V, at H 12, R 192, D_nope 48, D_rope 24, D_v 64:
     1537 keys: B 1, 1 query 16 / 24, 16 queries 21 / 25, 32 26 / 25; B 8: 18 / 54, 40 / 54, 55 / 54;
       B 2 and 4, 32 queries: 36 / 31, 40 / 38;
-    600 keys: B 4, 1 query 16 / 25, 16 queries 25 / 25; B 8, 16 queries 30 / 33;
-    300 keys: B 1, 16 queries 18 / 19; B 8, 8 queries 21 / 26, 16 28 / 26, 32 37 / 26;
-    128 keys: B 1, 1 query 16 / 14, 4 queries 17 / 14; B 8: 16 / 16, 18 / 16; B 32: 17 / 26, 24 / 26, 16
-      queries 51 / 26;
-    16 keys: 1 query, B 1 13 / 12, B 32 16 / 19; B 32, 16 queries 46 / 18.
+    600 keys: B 4, 1 query 16 / 25, 16 queries 25 / 25; B 8, 16 queries 30 / 33; B 32, 16 queries 66 / 74;
+    300 keys: B 1, 16 queries 18 / 19; B 4, 24 queries 25 / 21; B 8, 8 queries 21 / 26, 16 28 / 26, 32 37 / 26;
+    128 keys: B 1, 1 query 16 / 14, 16 queries 18 / 14; B 8, 16 queries 25 / 16; B 32: 17 / 26, 4 queries
+      24 / 26, 16 queries 51 / 26;
+    16 keys: 1 query, B 1 13 / 12, B 32 16 / 19; 16 queries, B 1 17 / 12, B 8 22 / 13, B 32 46 / 18.
     At H 32, R 256, D_nope 128, D_rope 64, D_v 128: 4096 keys, B 4, 32 queries 109 / 355; 300 keys, B 8,
-    8 queries 43 / 56, 16 queries 71 / 55.  (Up to 128 keys and few batches the K and V path, one launch
-    less there, is up to 3 us faster; the latent rows keep v exact: error against float64
-    1.7e-3, with K and V 2.1e-3.)"""
+    8 queries 43 / 56, 16 queries 71 / 55."""
     heads = D_nope + D_v
     pays = S_q * (24 * R * heads + S_kv * (3 * R - heads - D_nope)) <= S_kv * R * heads
-    return S_q <= 32 and (S_q == 1 or pays)
+    return S_q <= 32 and (S_q == 1 or B * H * S_q <= 768 or pays)
 
 
 def _head_rows(w: torch.Tensor) -> bool:
@@ -165,10 +166,10 @@ def _forward(ts, bc: int, softmax_scale: float, is_causal: bool, q_start: int, w
     """dsmoe_mla_attn_fwd (or _fwd_lse) over the batch chunks: bf16 out, the
     fp32 lse (None unless asked for) and the workspace, which holds the last
     chunk's K and V; None for a few queries, whose attention builds neither."""
-    if _few(ts[0].size(2), *ts[2].shape[1:], ts[0].size(3), ts[5].size(1)):
+    B, H, S_q, D_nope = ts[0].shape
+    if _few(min(B, bc), H, S_q, *ts[2].shape[1:], D_nope, ts[5].size(1)):
         return (*_forward_few(ts, bc, softmax_scale, is_causal, q_start), None)
     q_nope, q_pe, ctx_kv, ctx_pe, wkv_b_k, wkv_b_v = ts
-    B, H, S_q, _ = q_nope.shape
     D_v = wkv_b_v.size(1)
     dev = q_nope.device
     lib = L.load()

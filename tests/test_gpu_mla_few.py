@@ -25,12 +25,12 @@ def test_the_rule_chooses_the_path():
     """mla_attention takes the path that _few names: the C function it calls."""
     import dsmoe._lib as L
     import dsmoe.mla as M
-    for S_q, S_kv in ((1, 16), (4, 16), (10, 300), (12, 300), (33, 4096)):
-        ts, sc = _inputs(1, 2, S_q, S_kv, 192, 48, 24, 64, seed=S_q)
+    for B, S_q, S_kv in ((1, 1, 16), (1, 32, 16), (8, 8, 16), (8, 9, 16), (8, 16, 600), (1, 33, 4096)):
+        ts, sc = _inputs(B, 12, S_q, S_kv, 192, 48, 24, 64, seed=S_q)
         lib = mock.Mock(wraps=L.load())
         with mock.patch.object(L, "load", lambda: lib):
             M.mla_attention(*ts, sc, is_causal=False, q_start=0)
-        assert lib.dsmoe_mla_attn_few.called == M._few(S_q, S_kv, 192, 48, 64)
+        assert lib.dsmoe_mla_attn_few.called == M._few(B, 12, S_q, S_kv, 192, 48, 64)
         assert lib.dsmoe_mla_attn_few.called != lib.dsmoe_mla_attn_fwd_heads.called
     torch.cuda.synchronize()
 
@@ -109,7 +109,7 @@ def test_key_ranges(B, H, S_q, S_kv, R, Dn, Dr, Dv, causal, q_start):
     import dsmoe._lib as L
     import dsmoe.mla as M
     ts, sc = _inputs(B, H, S_q, S_kv, R, Dn, Dr, Dv, seed=S_q)
-    assert not M._few(S_q, S_kv, R, Dn, Dv)
+    assert not M._few(B, H, S_q, S_kv, R, Dn, Dv)
     w = torch.cat([ts[4], ts[5]], 1)
     ins, bc = M._prepare(*ts[:4], w[:, :Dn], w[:, Dn:])
     out, lse, ws = M._forward(ins, bc, sc, causal, q_start, want_lse=True)

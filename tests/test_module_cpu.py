@@ -316,11 +316,13 @@ def test_mla_operator_rejects_host_tensors_and_bad_dims():
         _check_mla_dim_limits(300, 8, 8, 8)
 
 
-@pytest.mark.parametrize("S_kv,most", [(16, 1), (33, 1), (64, 2), (128, 4), (300, 10), (600, 16), (1537, 28), (4096, 32)])
-def test_attention_takes_the_latent_rows_up_to(S_kv, most):
-    """dsmoe.mla._few at the 422m widths: queries over S_kv keys on the latent rows, more than `most` on K and V."""
+@pytest.mark.parametrize("B,S_kv,most", [(1, 16, 32), (2, 16, 32), (4, 16, 16), (8, 300, 10), (8, 16, 8), (32, 16, 2),
+                                         (32, 128, 4), (32, 600, 16), (32, 1537, 28), (32, 4096, 32), (100, 16, 1)])
+def test_attention_takes_the_latent_rows_up_to(B, S_kv, most):
+    """dsmoe.mla._few at the 422m widths: queries of B batches over S_kv keys on the latent rows, more than `most` on K
+    and V."""
     from dsmoe.mla import _few
-    assert [q for q in range(1, 65) if _few(q, S_kv, 192, 48, 64)] == list(range(1, most + 1))
+    assert [q for q in range(1, 65) if _few(B, 12, q, S_kv, 192, 48, 64)] == list(range(1, most + 1))
 
 
 def test_without_the_host_module_the_operators_serve_layer_calls(monkeypatch, recwarn):
